@@ -192,14 +192,14 @@ struct Batch final : BatchBase {
     const int n = int(b->runs.size());
     h_runs.resize(size_t(n));
     for (int r = 0; r < n; ++r) h_runs[r] = describe(b->runs[r]);
-    // the y/z march segment follows the march threads of the whole batch per direction
+    // the y/z march segment follows the march work of the whole batch per direction
     for (int d = 1; d < 3; ++d) {
-      long long threads = 0;
+      std::vector<fluxk::MarchShape> shapes;
       for (int r = 0; r < n; ++r) {
         const FluxArgsT<T> &a = h_runs[r].flux[0][0][d];
-        if (d < h_runs[r].ndir) threads += fluxk::march_threads(a.il, a.iu, a.jl, a.ju, a.kl, a.ku, d, fluxk::SEG);
+        if (d < h_runs[r].ndir) shapes.push_back(fluxk::march_shape(a.il, a.iu, a.jl, a.ju, a.kl, a.ku, d));
       }
-      const int seg = fluxk::march_seg(threads);
+      const int seg = fluxk::march_seg(shapes.data(), int(shapes.size()));
       for (int r = 0; r < n; ++r)
         for (auto &row : h_runs[r].flux)
           for (auto &ws : row) ws[d].seg = seg;

@@ -134,7 +134,8 @@ struct chq_ctx {
     if (d == 1) ju = g.je + 1; else if (g.two_d) { jl = g.js - 1; ju = g.je + 1; }
     if (d == 2) ku = g.ke + 1; else if (g.three_d) { kl = g.ks - 1; ku = g.ke + 1; }
     a.il = il; a.iu = iu; a.jl = jl; a.ju = ju; a.kl = kl; a.ku = ku;
-    a.seg = d == 0 ? fluxk::SEG : fluxk::march_seg(fluxk::march_threads(il, iu, jl, ju, kl, ku, d, fluxk::SEG));
+    const fluxk::MarchShape ms = fluxk::march_shape(il, iu, jl, ju, kl, ku, d);
+    a.seg = d == 0 ? 1 : fluxk::march_seg(&ms, 1);   // (x faces do not march)
     if (d == 0) { a.q1 = fast_div(g.ni); a.q2 = fast_div(ju - jl + 1); }
     else { a.q1 = fast_div(iu - il + 1); a.q2 = fast_div(d == 1 ? ku - kl + 1 : ju - jl + 1); }
     a.w = f64.w[wset];

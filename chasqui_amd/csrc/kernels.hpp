@@ -187,21 +187,47 @@ inline __host__ __device__ long long bc_points(const Geom &g, int d) {
 // of the lanes idle)
 namespace fluxk {
 constexpr int BX = 64, BY = 4;
-// Faces per thread in the y/z march. SEG where the launch's march threads fill the device
-// (measured at 256^3: 24 beats 8, 16, 32 in FP64 and 13, 20, 26, 37, 52 in FP32); SEG_SMALL
-// where they would leave it idle (small meshes, batches of small runs), and SEG_TINY where
-// they would use a sixteenth of it, since one thread's serial march is then the launch's
-// latency. The choice moves work between threads only: every
-// face is computed by the same expressions either way.
-constexpr int SEG = 24, SEG_SMALL = 8, SEG_TINY = 4;
-constexpr long long SEG_FILL = 131072;   // march threads of two 256-thread blocks per CU, 256 CUs
-// march threads of direction d (1 or 2) for segments of `seg` faces, from the face ranges
-inline __host__ __device__ long long march_threads(int il, int iu, int jl, int ju, int kl, int ku, int d, int seg) {
-  const long long nx = iu - il + 1, nt = d == 1 ? ku - kl + 1 : ju - jl + 1, nd = d == 1 ? ju - jl + 1 : ku - kl + 1;
-  return nx * nt * ((nd + seg - 1) / seg);
+// Faces per thread in the y/z march. A thread of a segment of s faces reconstructs s + 1 cells and
+// solves s faces one after the other: long segments save the extra reconstruction, short ones
+// give a small launch more waves and a shorter serial chain. march_seg picks the candidate of
+// least cost (s + 0.7) (0.1 + 0.9 m), where m is the launch's 256-thread blocks per CU (a block
+// puts one wave on each SIMD of its CU, and the waves of a SIMD share its issue slots, so the
+// second block of a CU adds nine tenths of the first one's time); a partial last block per CU
+// counts three quarters of a whole one. The three constants are fitted to sweeps of the RK step
+// over segments of 1 to 32 on 64^2 .. 1024^2 and 32^3 .. 192^3, PLM, PPM, PPMX, WENO-Z and
+// characteristic PPMX, both precisions: the choice is within 0.5% of the best candidate on
+// average (5% at worst). Before (24 faces where the march threads fill the device, 8 below, 4
+// below a sixteenth of it), ms per RK3 step: 150x129 PPMX FP64 0.233 (now 0.187), 64x56x45 PPM
+// FP64 0.495 (0.396), 512^2 PPMX mixed 0.298 (0.258), 80x72x64 characteristic 1.089 (the same segment),
+// 128^3 PPM FP64 2.301 (2.249). The choice moves work between threads only: every face is
+// computed by the same expressions either way.
+struct MarchShape {
+  long long rows;   // threads per segment layer: the face range across the march direction
+  int nd;           // faces along it
+};
+// the march of direction d (1 or 2) over a face range
+inline MarchShape march_shape(int il, int iu, int jl, int ju, int kl, int ku, int d) {
+  const long long nx = iu - il + 1;
+  return d == 1 ? MarchShape{nx * (ku - kl + 1), ju - jl + 1} : MarchShape{nx * (ju - jl + 1), ku - kl + 1};
 }
-inline __host__ __device__ int march_seg(long long threads_at_seg) {
-  return threads_at_seg < SEG_FILL / 16 ? SEG_TINY : threads_at_seg < SEG_FILL ? SEG_SMALL : SEG;
+// the segment of a launch that marches `n` shapes (the runs of a batch; one for a single mesh)
+inline int march_seg(const MarchShape *sh, int n) {
+  static constexpr int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
+  int best = 1;
+  double least = 1e300;
+  for (const int s : cand) {
+    long long blocks = 0;
+    int len = 1;   // the longest serial march
+    for (int q = 0; q < n; ++q) {
+      blocks += (sh[q].rows * ((sh[q].nd + s - 1) / s) + 255) / 256;
+      len = len > sh[q].nd ? len : sh[q].nd;
+    }
+    const double per = double(blocks) / 256.0;   // 256 CUs
+    const double m = 0.75 * double((blocks + 255) / 256) + 0.25 * per;
+    const double cost = ((s < len ? s : len) + 0.7) * (0.1 + 0.9 * (m > 1.0 ? m : 1.0));
+    if (cost < least) { least = cost; best = s; }
+  }
+  return best;
 }
 
 template <Recon RC> constexpr bool wide_v = !(RC == Recon::dc || RC == Recon::plm);
