@@ -4,7 +4,7 @@
 // their launch descriptions (RunArgs) and the (run, tile) work lists of each kernel class.
 //
 // One RK step is the same kernel sequence as a single context's fused step, each launch
-// covering every run: flux x1..x3, corner EMF, update, boundaries, con2prim (+ fofc list),
+// covering every run: flux x1..x3, corner EMF, update, ghost fill + con2prim (+ fofc list),
 // then the fofc branch over the runs that flagged cells (compacted on the device), then the
 // control-block updates (per-run dt, t, cycle, primitive-set flip). No reduction spans runs,
 // so every run's result is bitwise the one it gets alone.
@@ -135,27 +135,12 @@ struct Batch final : BatchBase {
         a.flag_mode = c->cfg.fofc ? 2 : 0;
         r.c2p[buf][ws] = a;
       }
-    for (int buf = 0; buf < 2; ++buf)
-      for (int d = 0; d < 3; ++d) {
-        BcArgs a{};
-        a.g = c->g;
-        a.nvar = 5;
-        a.u = c->u[buf];
-        a.b1 = c->bf[buf][0]; a.b2 = c->bf[buf][1]; a.b3 = c->bf[buf][2];
-        a.ctrl = k;
-        a.only_if_bad = 0;
-        a.bc = c->cfg.bc[d];
-        r.bc[buf][d] = a;
-      }
     r.ctrl = k;
     r.badlist = c->badlist;
     r.ndir = c->ndir();
     const Geom &g = c->g;
     r.cond_tiles[0] = update_vb(g).n;
-    r.cond_tiles[1] = int((bc_points(g, 0) + 255) / 256);
-    r.cond_tiles[2] = g.two_d ? int((bc_points(g, 1) + 255) / 256) : 0;
-    r.cond_tiles[3] = g.three_d ? int((bc_points(g, 2) + 255) / 256) : 0;
-    r.cond_tiles[4] = c2p_vb(g).n;
+    r.cond_tiles[1] = ghost_tiles(g) + active_vb(g).n;
     return r;
   }
 
@@ -179,10 +164,8 @@ struct Batch final : BatchBase {
     switch (k) {
       case K_CORNER: return corner_vb(g).n;
       case K_UPDATE: return update_vb(g).n;
-      case K_BC1: return int((bc_points(g, 0) + 255) / 256);
-      case K_BC2: return g.two_d ? int((bc_points(g, 1) + 255) / 256) : 0;
-      case K_BC3: return g.three_d ? int((bc_points(g, 2) + 255) / 256) : 0;
-      default: return c2p_vb(g).n;
+      case K_C2P: return ghost_tiles(g) + active_vb(g).n;
+      default: return 0;   // K_BC1..3: the ghost fill is part of con2prim's launch
     }
   }
 
@@ -252,7 +235,7 @@ struct Batch final : BatchBase {
     return CHQ_OK;
   }
 
-  // The launches of a stage; flux and boundary classes that no run of the batch has (the y and z
+  // The launches of a stage; flux classes that no run of the batch has (the y and z
   // directions of 1D runs, z of 2D) are left out (present[], fixed when the step is enqueued or
   // captured; a change re-captures the graph). The control launches between stages are merged:
   // begin step + begin stage 1, end stage + begin next, end last stage + end step.
@@ -267,8 +250,6 @@ struct Batch final : BatchBase {
       if (present[K_FLUX1 + d]) HIPCHK(launchb_flux(d_runs, list(K_FLUX1 + d), d, cf.cur, rc, rs, g[K_FLUX1 + d], st));
     HIPCHK(launchb_corner<T>(d_runs, list(K_CORNER), g[K_CORNER], st));
     HIPCHK(launchb_update<T>(d_runs, list(K_UPDATE), cf.out, cf.g0, cf.g1, cf.beta, g[K_UPDATE], st));
-    for (int d = 0; d < 3; ++d)
-      if (present[K_BC1 + d]) HIPCHK(launchb_bc<T>(d_runs, list(K_BC1 + d), d, cf.out, g[K_BC1 + d], st));
     HIPCHK(launchb_c2p<T>(d_runs, list(K_C2P), cf.out, last, g[K_C2P], st));
     // fofc branch of the runs that flagged cells: for batches of small runs, one block per run
     // in two launches; otherwise compacted over the flagged runs, one launch per class
@@ -280,8 +261,6 @@ struct Batch final : BatchBase {
       HIPCHK(launchb_repair(d_runs, cond(), cf.cur, g[G_REPAIR], st));
       HIPCHK(launchb_corner_cond<T>(d_runs, cond(), g[G_REPAIR], st));
       HIPCHK(launchb_update_cond<T>(d_runs, cond(), cf.out, cf.g0, cf.g1, cf.beta, g[G_COND], st));
-      for (int d = 0; d < 3; ++d)
-        if (present[K_BC1 + d]) HIPCHK(launchb_bc_cond<T>(d_runs, cond(), d, cf.out, g[G_COND], st));
       HIPCHK(launchb_c2p_cond<T>(d_runs, cond(), cf.out, last, g[G_COND], st));
     }
     if (last) return ctrl(CTRL_END_LAST, 0);
@@ -302,14 +281,14 @@ struct Batch final : BatchBase {
   bool small_branch = false;
   unsigned captured_present = ~0u;
   // the runs' fofc branch fits one block each: at most SMALL_BRANCH_TILES tiles of re-update,
-  // boundaries and con2prim per run (a few thousand cells), where launches cost more than the
+  // ghost fill and con2prim per run (a few thousand cells), where launches cost more than the
   // block's serial walk over its tiles
   static constexpr int SMALL_BRANCH_TILES = 48;
   bool small_runs() const {
     if (h_runs.empty()) return false;
     for (const RunArgs<T> &r : h_runs) {
       int t = 0;
-      for (int q = 0; q < 5; ++q) t += r.cond_tiles[q];
+      for (int q = 0; q < 2; ++q) t += r.cond_tiles[q];
       if (t > SMALL_BRANCH_TILES) return false;
     }
     return true;
@@ -333,7 +312,6 @@ struct Batch final : BatchBase {
         break;
       case K_CORNER: HIPCHK(launchb_corner<T>(d_runs, list(q), gsz, st)); break;
       case K_UPDATE: HIPCHK(launchb_update<T>(d_runs, list(q), 1, 1.0, 0.0, 1.0, gsz, st)); break;
-      case K_BC1: case K_BC2: case K_BC3: HIPCHK(launchb_bc<T>(d_runs, list(q), q - K_BC1, 1, gsz, st)); break;
       case K_C2P: HIPCHK(launchb_c2p<T>(d_runs, list(q), 1, 0, gsz, st)); break;
       default: break;
     }

@@ -502,10 +502,8 @@ int sts_bc(chq_ctx *c, Ctrl *k, double *u, double *const b[3]) {
   a.b1 = b[0]; a.b2 = b[1]; a.b3 = b[2];
   a.ctrl = k;
   a.only_if_bad = 0;
-  a.bc = c->cfg.bc[0];
-  HIPCHK(launch_bc(a, 0, c->stream));
-  if (c->g.two_d) { a.bc = c->cfg.bc[1]; HIPCHK(launch_bc(a, 1, c->stream)); }
-  if (c->g.three_d) { a.bc = c->cfg.bc[2]; HIPCHK(launch_bc(a, 2, c->stream)); }
+  for (int d = 0; d < 3; ++d) a.bc[d] = c->cfg.bc[d];
+  HIPCHK(launch_fill(a, c->stream));
   return CHQ_OK;
 }
 
@@ -794,22 +792,25 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
     HIPCHK(launch_flag(fl, c->stream));
   }
   const int first = strict ? 2 : adaptive ? 4 : 0;
-  c->tmark(CHQ_K_BC, true);
-  HIPCHK(c->boundaries(cf.out, nvar, k, first));
-  c->tmark(CHQ_K_BC, false);
+  // the ghost fill is part of the con2prim launch unless entropy is transported (dual energy's
+  // con2prim rewrites u, which the fill of another block would be reading)
+  if (c->entropy) {
+    c->tmark(CHQ_K_BC, true);
+    HIPCHK(c->boundaries(cf.out, nvar, k, first));
+    c->tmark(CHQ_K_BC, false);
+  }
   C2pArgsT<T> ca = c->c2p_args_t(fs, cf.out, wn, k);
   ca.only_if_bad = first;
   ca.write_went = c->entropy;
-  // u[IENT] is read by nothing in this path unless entropy is transported: the intermediate RK
-  // states never resynchronise it, and the last stage leaves it to sync_ient (the first host
-  // read of the state or per-kernel entry point), which stores what this con2prim would have
-  ca.entropy_out = c->entropy;
+  // u[IENT] is read by nothing in this path unless entropy is transported: launch_fill_c2p leaves
+  // it alone, and that of the final state to sync_ient (the first host read of the state or
+  // per-kernel entry point), which stores what con2prim would have
   if (last && !c->entropy) c->ient_stale = true;   // the last stage writes buffer 0
   ca.compute_dt = last && !(c->cfg.sts || c->cfg.cooling);   // split steps take dt after the splits
   ca.slot = 0;
   ca.flag_mode = adaptive ? 3 : 0;
   c->tmark(CHQ_K_C2P, true);
-  HIPCHK(launch_c2p<T>(ca, c->stream));
+  HIPCHK(c->entropy ? launch_c2p<T>(ca, c->stream) : launch_fill_c2p<T>(ca, c->stream));
   c->tmark(CHQ_K_C2P, false);
   if (c->cfg.fofc) {
     c->tmark(CHQ_K_REPAIR, true);
@@ -834,12 +835,12 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
       sb.only_if_bad = 1;
       HIPCHK(launch_gravity(sb, c->stream));
     }
-    HIPCHK(c->boundaries(cf.out, nvar, k, 1));
+    if (c->entropy) HIPCHK(c->boundaries(cf.out, nvar, k, 1));
     C2pArgsT<T> cb = ca;
     cb.flag_mode = 0;
     cb.slot = 1;
     cb.only_if_bad = 1;   // (after ca's gate 2: exactly one of the two runs)
-    HIPCHK(launch_c2p<T>(cb, c->stream));
+    HIPCHK(c->entropy ? launch_c2p<T>(cb, c->stream) : launch_fill_c2p<T>(cb, c->stream));
     c->tmark(CHQ_K_REPAIR, false);
   }
   return CHQ_OK;

@@ -183,8 +183,8 @@ struct chq_ctx {
     a.b1 = bf[buf][0]; a.b2 = bf[buf][1]; a.b3 = bf[buf][2];
     a.u = u[buf];
     a.w = f64.w[wset]; a.bcc = f64.bcc[wset]; a.ecc = f64.ecc[wset];
+    for (int d = 0; d < 3; ++d) a.bc[d] = cfg.bc[d];
     a.write_went = 1;
-    a.entropy_out = 1;
     a.flag = flag;
     a.badlist = badlist;
     a.ctrl = c;
@@ -198,12 +198,8 @@ struct chq_ctx {
     a.b1 = bf[buf][0]; a.b2 = bf[buf][1]; a.b3 = bf[buf][2];
     a.ctrl = c;
     a.only_if_bad = only_if_bad;
-    a.bc = cfg.bc[0];
-    hipError_t e = launch_bc(a, 0, stream);
-    if (e != hipSuccess) return e;
-    if (g.two_d) { a.bc = cfg.bc[1]; e = launch_bc(a, 1, stream); if (e != hipSuccess) return e; }
-    if (g.three_d) { a.bc = cfg.bc[2]; e = launch_bc(a, 2, stream); }
-    return e;
+    for (int d = 0; d < 3; ++d) a.bc[d] = cfg.bc[d];
+    return launch_fill(a, stream);
   }
   int ndir() const { return 1 + (g.two_d ? 1 : 0) + (g.three_d ? 1 : 0); }
   bool diffusive() const { return cfg.nu > 0.0 || cfg.kappa > 0.0 || cfg.eta > 0.0; }
@@ -301,7 +297,8 @@ struct chq_ctx {
     C2pArgsT<T> a{};
     a.g = a0.g; a.eos = a0.eos; a.b1 = a0.b1; a.b2 = a0.b2; a.b3 = a0.b3; a.u = a0.u;
     a.w = f.w[wset]; a.bcc = f.bcc[wset]; a.ecc = f.ecc[wset];
-    a.write_went = 1; a.entropy_out = 1; a.compute_dt = 0; a.slot = 0; a.flag_mode = 0;
+    for (int d = 0; d < 3; ++d) a.bc[d] = cfg.bc[d];
+    a.write_went = 1; a.compute_dt = 0; a.slot = 0; a.flag_mode = 0;
     a.flag = flag; a.badlist = badlist; a.ctrl = c; a.only_if_bad = 0;
     a.xg = XG_C2P;
     return a;

@@ -9,6 +9,7 @@
 #include <type_traits>
 
 #include "common.hpp"
+#include "ghost.hpp"
 
 namespace chq {
 
@@ -95,9 +96,10 @@ struct UpdateArgsT {
 };
 using UpdateArgs = UpdateArgsT<double>;
 
+// the ghost fill of all directions (bc[d]: 0 periodic, 1 outflow, 2 reflecting)
 struct BcArgs {
   Geom g;
-  int bc, nvar;
+  int bc[3], nvar;
   double *u, *b1, *b2, *b3;
   const Ctrl *ctrl;
   int only_if_bad;
@@ -108,11 +110,11 @@ template <class T>
 struct C2pArgsT {
   Geom g;
   Eos eos;
-  const double *b1, *b2, *b3;
+  double *b1, *b2, *b3;        // (the fused ghost fill writes their ghost entries)
   double *u;
   T *w, *bcc, *ecc;
+  int bc[3];                   // boundary conditions of the fused ghost fill
   int write_went;              // also store w[IENT] (needed when entropy is transported)
-  int entropy_out;             // resynchronise u[IENT] = rho p / rho^gamma
   int compute_dt;
   int slot;                    // which running minimum receives the CFL dt (0 or 1)
   int flag_mode;               // 0: none; 1: flag array + count; 2: append flagged cells to badlist
@@ -174,11 +176,9 @@ inline __host__ __device__ VB update_vb(const Geom &g) {
 }
 // con2prim: every cell, ghosts included
 inline __host__ __device__ VB c2p_vb(const Geom &g) { return vgrid(g.ni, g.nj, g.nk); }
-// boundaries of direction d: threads over (k, j, ghost), (k, ghost, i) or (ghost, j, i)
-inline __host__ __device__ long long bc_points(const Geom &g, int d) {
-  if (d == 0) return (long long)(g.nk + 1) * (g.nj + 1) * g.ng;
-  if (d == 1) return (long long)(g.nk + 1) * g.ng * (g.ni + 1);
-  return (long long)g.ng * (g.nj + 1) * (g.ni + 1);
+// con2prim with the fused ghost fill: the active cells, in tiles after those of the ghost points
+inline __host__ __device__ VB active_vb(const Geom &g) {
+  return vgrid(g.ie - g.is + 1, g.je - g.js + 1, g.ke - g.ks + 1);
 }
 
 // face-flux decomposition (flux_impl.hpp): x faces by wave64 windows over the rows' cells laid
@@ -290,16 +290,15 @@ struct RunArgs {
   CornerArgsT<T> corner[2];      // [primitive set]
   UpdateArgsT<T> update[2];      // [output buffer]; coefficients come with the launch
   C2pArgsT<T> c2p[2][2];         // [buffer][primitive set written]
-  BcArgs bc[2][3];               // [buffer][dir]
   Ctrl *ctrl;
   int *badlist;                  // cells flagged by con2prim in the current stage
   int ndir;
-  int cond_tiles[5];             // tiles of the whole-mesh fofc re-runs: update, bc x1..x3, c2p
+  int cond_tiles[2];             // tiles of the whole-mesh fofc re-runs: update, ghost fill + con2prim
 };
 
 // The fofc branch of a batch: the runs that flagged cells in the current stage, compacted on
 // the device, with per-class tile prefixes (classes below).
-enum : int { CL_REPAIR = 0, CL_CORNER, CL_UPDATE, CL_BC1, CL_BC2, CL_BC3, CL_C2P, CL_N };
+enum : int { CL_REPAIR = 0, CL_CORNER, CL_UPDATE, CL_C2P, CL_N };
 struct CondList {
   int cap;             // capacity in runs
   int *base;           // [0] = number of flagged runs, then run[cap], then pre[CL_N][cap + 1]
@@ -327,7 +326,7 @@ hipError_t launch_ient_sync(const C2pArgsT<double> &a, hipStream_t s);
 // (flagged) cell with the control block's epoch, then recompute exactly the stamped points
 hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, int *marks, hipStream_t s);
 template <class T> hipError_t launch_update_near(const UpdateArgsT<T> &a, const int *marks, hipStream_t s);
-hipError_t launch_bc(const BcArgs &a, int dir, hipStream_t s);
+hipError_t launch_fill(const BcArgs &a, hipStream_t s);
 
 // explicit diffusion (FP64 single-mesh path), diffusion.hip
 struct DiffArgs {
@@ -376,6 +375,8 @@ hipError_t launch_limit_fluxes(const SrcArgs &a, int dir, hipStream_t s);
 hipError_t launch_gravity(const SrcArgs &a, hipStream_t s);
 hipError_t launch_cooling(const SrcArgs &a, hipStream_t s);
 template <class T> hipError_t launch_c2p(const C2pArgsT<T> &a, hipStream_t s);
+// ghost fill and con2prim of every cell in one launch (u[IENT] neither transported nor stored)
+template <class T> hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s);
 hipError_t launch_flag(const C2pArgs &a, hipStream_t s);   // standalone FlagBadCells
 // control-block kernels
 hipError_t launch_ctrl_begin_step(Ctrl *c, hipStream_t s);
@@ -398,12 +399,10 @@ template <class T> hipError_t launchb_fofc_runs(const RunArgs<T> *R, const int *
                                                 double g1, double beta, int last, hipStream_t s);
 template <class T> hipError_t launchb_corner(const RunArgs<T> *R, ItemList L, int grid, hipStream_t s);
 template <class T> hipError_t launchb_update(const RunArgs<T> *R, ItemList L, int out, double g0, double g1, double beta, int grid, hipStream_t s);
-template <class T> hipError_t launchb_bc(const RunArgs<T> *R, ItemList L, int dir, int buf, int grid, hipStream_t s);
 template <class T> hipError_t launchb_c2p(const RunArgs<T> *R, ItemList L, int buf, int last, int grid, hipStream_t s);
 template <class T> hipError_t launchb_fofc_scan(const RunArgs<T> *R, const int *nruns, CondList C, hipStream_t s);
 template <class T> hipError_t launchb_corner_cond(const RunArgs<T> *R, CondList C, int grid, hipStream_t s);
 template <class T> hipError_t launchb_update_cond(const RunArgs<T> *R, CondList C, int out, double g0, double g1, double beta, int grid, hipStream_t s);
-template <class T> hipError_t launchb_bc_cond(const RunArgs<T> *R, CondList C, int dir, int buf, int grid, hipStream_t s);
 template <class T> hipError_t launchb_c2p_cond(const RunArgs<T> *R, CondList C, int buf, int last, int grid, hipStream_t s);
 // control-block step of every run (one thread per table slot, `cap` slots); the end of a step
 // also writes live[r] = run r has not reached tlim / nlim

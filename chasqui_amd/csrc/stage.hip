@@ -536,159 +536,40 @@ __global__ void __launch_bounds__(256) k_update_march(const UpdateArgsT<T> a, co
 }
 
 // ---------------------------------------------------------------- boundaries
-// physics.hpp:354-432. x1: threads over (k, j, g) with g fastest; x2: (k, g, i); x3: (g, j, i).
-__device__ __forceinline__ void bc1_at(const BcArgs &a, const long long t) {
-  const Geom &g = a.g;
-  const int ng = g.ng;
-  const long long n_all = (long long)(g.nk + 1) * (g.nj + 1) * ng;
-  if (t >= n_all) return;
-  const int gg = int(t % ng), j = int((t / ng) % (g.nj + 1)), k = int(t / ((long long)ng * (g.nj + 1)));
-  const int bc = a.bc, nx = g.nx1, is = g.is, ie = g.ie;
-  const int il = gg, ir = ie + 1 + gg;
-  const int sl = bc == 0 ? il + nx : bc == 1 ? is : 2 * is - 1 - il;
-  const int sr = bc == 0 ? ir - nx : bc == 1 ? ie : 2 * ie + 1 - ir;
-  const double sg = bc == 2 ? -1.0 : 1.0;
-  const long long row = g.at(k, j, 0), cs = g.cstride;
-  // every load of this thread first, then every store: none of its stores feeds one of its
-  // loads, and its two ghosts of each row lie in lines of their own, so the loads overlap
-  const bool cells = k < g.nk && j < g.nj;
-  double vl[NVAR], vr[NVAR], b2l = 0.0, b2r = 0.0, b3l = 0.0, b3r = 0.0;
-  if (cells) {
+// one thread per ghost point (ghost.hpp)
+
+// fill one ghost point: face fields and, if it is a cell, `nvar` conserved values into uv
+__device__ __forceinline__ void fill_point(const Geom &g, const int *bc, int nvar, double *u, double *b1, double *b2,
+                                           double *b3, int k, int j, int i, double *uv) {
+  const long long c = g.at(k, j, i), cs = g.cstride;
+  bool o1, o2, o3;
+  const double v1 = ghost_face<1>(g, bc, b1, k, j, i, o1), v2 = ghost_face<2>(g, bc, b2, k, j, i, o2),
+               v3 = ghost_face<3>(g, bc, b3, k, j, i, o3);
+  if (k < g.nk && j < g.nj && i < g.ni) {
+    int sk = k, sj = j, si = i;
+    const int m = ghost_source<0>(g, bc, sk, sj, si);
+    const double *us = u + g.at(sk, sj, si);
 #pragma unroll
     for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) { vl[n] = a.u[n * cs + row + sl]; vr[n] = a.u[n * cs + row + sr]; }
-    b2l = a.b2[row + sl]; b2r = a.b2[row + sr];
-    b3l = a.b3[row + sl]; b3r = a.b3[row + sr];
-  }
-  double *b1 = a.b1 + row;
-  const int fl = gg, fr = ie + 2 + gg;
-  double f1l, f1r;
-  if (bc == 0) { f1l = b1[fl + nx]; f1r = b1[fr - nx]; }
-  else if (bc == 1) { f1l = b1[is]; f1r = b1[ie + 1]; }
-  else { f1l = -b1[2 * is - fl]; f1r = -b1[2 * (ie + 1) - fr]; }
-  const bool shared = bc == 0 && gg == 0;   // the periodic shared face takes the lower copy
-  const double f1s = shared ? b1[is] : 0.0;
-  if (cells) {
+      if (n < nvar) uv[n] = us[n * cs];
+    if (m & 1) uv[IM1] = -1.0 * uv[IM1];
+    if (m & 2) uv[IM2] = -1.0 * uv[IM2];
+    if (m & 4) uv[IM3] = -1.0 * uv[IM3];
 #pragma unroll
     for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) {
-        const double f = n == IM1 ? sg : 1.0;
-        a.u[n * cs + row + il] = f * vl[n];
-        a.u[n * cs + row + ir] = f * vr[n];
-      }
-    a.b2[row + il] = b2l; a.b2[row + ir] = b2r;
-    a.b3[row + il] = b3l; a.b3[row + ir] = b3r;
+      if (n < nvar) u[n * cs + c] = uv[n];
   }
-  b1[fl] = f1l;
-  b1[fr] = f1r;
-  if (shared) b1[ie + 1] = f1s;
+  if (!o1) b1[c] = v1;
+  if (!o2) b2[c] = v2;
+  if (!o3) b3[c] = v3;
 }
 
-__device__ __forceinline__ void bc2_at(const BcArgs &a, const long long t) {
-  const Geom &g = a.g;
-  const int ng = g.ng;
-  const long long n_all = (long long)(g.nk + 1) * ng * (g.ni + 1);
-  if (t >= n_all) return;
-  const int i = int(t % (g.ni + 1)), gg = int((t / (g.ni + 1)) % ng), k = int(t / ((long long)ng * (g.ni + 1)));
-  const int bc = a.bc, ny = g.nx2, js = g.js, je = g.je;
-  const int jl = gg, jr = je + 1 + gg;
-  const int sl = bc == 0 ? jl + ny : bc == 1 ? js : 2 * js - 1 - jl;
-  const int sr = bc == 0 ? jr - ny : bc == 1 ? je : 2 * je + 1 - jr;
-  const double sg = bc == 2 ? -1.0 : 1.0;
-  const long long sj = g.pitch, cs = g.cstride;
-  const long long col = g.at(k, 0, i);
-  // loads first, then stores (as in bc1_at)
-  const bool cells = k < g.nk && i < g.ni, faces1 = k < g.nk;
-  double vl[NVAR], vr[NVAR], b3l = 0.0, b3r = 0.0, b1l = 0.0, b1r = 0.0;
-  if (cells) {
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) { vl[n] = a.u[n * cs + col + sl * sj]; vr[n] = a.u[n * cs + col + sr * sj]; }
-    b3l = a.b3[col + sl * sj]; b3r = a.b3[col + sr * sj];
-  }
-  if (faces1) { b1l = a.b1[col + sl * sj]; b1r = a.b1[col + sr * sj]; }
-  double *b2 = a.b2 + col;
-  const int fl = gg, fr = je + 2 + gg;
-  double f2l, f2r;
-  if (bc == 0) { f2l = b2[(fl + ny) * sj]; f2r = b2[(fr - ny) * sj]; }
-  else if (bc == 1) { f2l = b2[js * sj]; f2r = b2[(je + 1) * sj]; }
-  else { f2l = -b2[(2 * js - fl) * sj]; f2r = -b2[(2 * (je + 1) - fr) * sj]; }
-  const bool shared = bc == 0 && gg == 0;
-  const double f2s = shared ? b2[js * sj] : 0.0;
-  if (cells) {
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) {
-        const double f = n == IM2 ? sg : 1.0;
-        a.u[n * cs + col + jl * sj] = f * vl[n];
-        a.u[n * cs + col + jr * sj] = f * vr[n];
-      }
-    a.b3[col + jl * sj] = b3l; a.b3[col + jr * sj] = b3r;
-  }
-  if (faces1) { a.b1[col + jl * sj] = b1l; a.b1[col + jr * sj] = b1r; }
-  b2[fl * sj] = f2l;
-  b2[fr * sj] = f2r;
-  if (shared) b2[(je + 1) * sj] = f2s;
-}
-
-__device__ __forceinline__ void bc3_at(const BcArgs &a, const long long t) {
-  const Geom &g = a.g;
-  const int ng = g.ng;
-  const long long n_all = (long long)ng * (g.nj + 1) * (g.ni + 1);
-  if (t >= n_all) return;
-  const int i = int(t % (g.ni + 1)), j = int((t / (g.ni + 1)) % (g.nj + 1)), gg = int(t / ((long long)(g.nj + 1) * (g.ni + 1)));
-  const int bc = a.bc, nz = g.nx3, ks = g.ks, ke = g.ke;
-  const int kl = gg, kr = ke + 1 + gg;
-  const int sl = bc == 0 ? kl + nz : bc == 1 ? ks : 2 * ks - 1 - kl;
-  const int sr = bc == 0 ? kr - nz : bc == 1 ? ke : 2 * ke + 1 - kr;
-  const double sg = bc == 2 ? -1.0 : 1.0;
-  const long long sk = g.plane, cs = g.cstride;
-  const long long col = g.at(0, j, i);
-  // loads first, then stores (as in bc1_at)
-  const bool cells = j < g.nj && i < g.ni;
-  double vl[NVAR], vr[NVAR];
-  if (cells) {
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) { vl[n] = a.u[n * cs + col + sl * sk]; vr[n] = a.u[n * cs + col + sr * sk]; }
-  }
-  const double b1l = a.b1[col + sl * sk], b1r = a.b1[col + sr * sk];
-  const double b2l = a.b2[col + sl * sk], b2r = a.b2[col + sr * sk];
-  double *b3 = a.b3 + col;
-  const int fl = gg, fr = ke + 2 + gg;
-  double f3l, f3r;
-  if (bc == 0) { f3l = b3[(fl + nz) * sk]; f3r = b3[(fr - nz) * sk]; }
-  else if (bc == 1) { f3l = b3[ks * sk]; f3r = b3[(ke + 1) * sk]; }
-  else { f3l = -b3[(2 * ks - fl) * sk]; f3r = -b3[(2 * (ke + 1) - fr) * sk]; }
-  const bool shared = bc == 0 && gg == 0;
-  const double f3s = shared ? b3[ks * sk] : 0.0;
-  if (cells) {
-#pragma unroll
-    for (int n = 0; n < NVAR; ++n)
-      if (n < a.nvar) {
-        const double f = n == IM3 ? sg : 1.0;
-        a.u[n * cs + col + kl * sk] = f * vl[n];
-        a.u[n * cs + col + kr * sk] = f * vr[n];
-      }
-  }
-  a.b1[col + kl * sk] = b1l; a.b1[col + kr * sk] = b1r;
-  a.b2[col + kl * sk] = b2l; a.b2[col + kr * sk] = b2r;
-  b3[fl * sk] = f3l;
-  b3[fr * sk] = f3r;
-  if (shared) b3[(ke + 1) * sk] = f3s;
-}
-
-template <int DIR>
-__device__ __forceinline__ void bc_at(const BcArgs &a, const long long t) {
-  if (DIR == 0) bc1_at(a, t);
-  else if (DIR == 1) bc2_at(a, t);
-  else bc3_at(a, t);
-}
-
-template <int DIR>
-__global__ void __launch_bounds__(256) k_bc(const BcArgs a) {
+__global__ void __launch_bounds__(256) k_fill(const BcArgs a) {
   if (!gate(a.ctrl, a.only_if_bad)) return;
-  bc_at<DIR>(a, (long long)blockIdx.x * blockDim.x + threadIdx.x);
+  int k, j, i;
+  if (!ghost_point(a.g, int(blockIdx.x) * 256 + int(threadIdx.x), k, j, i)) return;
+  double uv[NVAR];
+  fill_point(a.g, a.bc, a.nvar, a.u, a.b1, a.b2, a.b3, k, j, i, uv);
 }
 
 // ---------------------------------------------------------------- reductions
@@ -707,21 +588,20 @@ __device__ __forceinline__ int wave_sum(int v) {
 // flag_mode 1 writes the flag array (reference semantics); 2 appends flagged cells to a list.
 // DT: reduce the CFL minimum. ENT: resynchronise u[IENT] (and w[IENT] if write_went); the
 // lean variant (no pow) serves RK stages whose u[IENT] nothing reads.
-// bz: the cell-centred x3 field (the caller averages the two x3 faces). DE: the dual
-// energy branches are compiled in (without them the kernel holds no pow() for the flag and
+// DE: the dual energy branches are compiled in (without them the kernel holds no pow() for the flag and
 // needs far fewer registers).
 // IENT_ONLY: store u[IENT] and nothing else (the deferred resynchronisation, k_ient_sync).
+// uv, bx, by, bz: the cell's five conserved values and cell-centred field, loaded by the caller;
+// c: where the primitives go.
 template <class T, bool DT, bool ENT, bool DE, bool IENT_ONLY = false>
-__device__ __forceinline__ void c2p_core(const C2pArgsT<T> &a, int k, int j, int i, const double bz, double &mdt,
+__device__ __forceinline__ void c2p_core(const C2pArgsT<T> &a, const long long c, const double *uv, const double bx,
+                                         const double by, const double bz, const bool active, double &mdt,
                                          int &nbad_local) {
   const Geom &g = a.g;
   const Eos e = a.eos;
-  const long long c = g.at(k, j, i), sj = g.pitch, cs = g.cstride;
-  const double bx = 0.5 * (a.b1[c] + a.b1[c + 1]);
-  const double by = g.two_d ? 0.5 * (a.b2[c] + a.b2[c + sj]) : a.b2[c];
+  const long long cs = g.cstride;
   double *u = a.u + c;
-  const double u0 = u[IDN * cs], u1 = u[IM1 * cs], u2 = u[IM2 * cs], u3 = u[IM3 * cs], u4 = u[IEN * cs];
-  const bool active = i >= g.is && i <= g.ie && j >= g.js && j <= g.je && k >= g.ks && k <= g.ke;
+  const double u0 = uv[IDN], u1 = uv[IM1], u2 = uv[IM2], u3 = uv[IM3], u4 = uv[IEN];
   // flag_mode 3: append (as 2) unless this stage already flagged before the fill
   const int fm = IENT_ONLY ? 0 : a.flag_mode == 3 ? (a.ctrl->early ? 0 : 2) : a.flag_mode;
   if (fm && active) {   // fofc.hpp:24-40 on the tentative state
@@ -792,9 +672,48 @@ __device__ __forceinline__ void c2p_core(const C2pArgsT<T> &a, int k, int j, int
 template <class T, bool DT, bool ENT, bool DE, bool IENT_ONLY = false>
 __device__ __forceinline__ void c2p_at(const C2pArgsT<T> &a, int k, int j, int i, double &mdt, int &nbad_local) {
   const Geom &g = a.g;
-  const long long c = g.at(k, j, i);
+  const long long c = g.at(k, j, i), cs = g.cstride;
+  const double bx = 0.5 * (a.b1[c] + a.b1[c + 1]);
+  const double by = g.two_d ? 0.5 * (a.b2[c] + a.b2[c + g.pitch]) : a.b2[c];
   const double bz = g.three_d ? 0.5 * (a.b3[c] + a.b3[c + g.plane]) : a.b3[c];
-  c2p_core<T, DT, ENT, DE, IENT_ONLY>(a, k, j, i, bz, mdt, nbad_local);
+  const double *u = a.u + c;
+  const double uv[5] = {u[IDN * cs], u[IM1 * cs], u[IM2 * cs], u[IM3 * cs], u[IEN * cs]};
+  const bool active = i >= g.is && i <= g.ie && j >= g.js && j <= g.je && k >= g.ks && k <= g.ke;
+  c2p_core<T, DT, ENT, DE, IENT_ONLY>(a, c, uv, bx, by, bz, active, mdt, nbad_local);
+}
+
+// Ghost fill and con2prim of tile `tile`: ghost points first (ghost_tiles), then the active
+// cells. A ghost cell is converted from the values it is filled with, read at their source, so
+// the launch needs no order between its tiles: active cells read active entries only (the upper
+// face of a periodic direction is read from its lower copy, which the fill writes there).
+template <class T, bool DT>
+__device__ __forceinline__ void fill_c2p_tile(const C2pArgsT<T> &a, const VB &v, int tile, int ngt, double &mdt) {
+  const Geom &g = a.g;
+  int k, j, i, nb = 0;
+  if (tile < ngt) {
+    if (!ghost_point(g, tile * 256 + int(threadIdx.x), k, j, i)) return;
+    double uv[NVAR];
+    fill_point(g, a.bc, 5, a.u, a.b1, a.b2, a.b3, k, j, i, uv);
+    if (k >= g.nk || j >= g.nj || i >= g.ni) return;
+    bool own;
+    const double bx = 0.5 * (ghost_face<1>(g, a.bc, a.b1, k, j, i, own) + ghost_face<1>(g, a.bc, a.b1, k, j, i + 1, own));
+    double by = ghost_face<2>(g, a.bc, a.b2, k, j, i, own), bz = ghost_face<3>(g, a.bc, a.b3, k, j, i, own);
+    if (g.two_d) by = 0.5 * (by + ghost_face<2>(g, a.bc, a.b2, k, j + 1, i, own));
+    if (g.three_d) bz = 0.5 * (bz + ghost_face<3>(g, a.bc, a.b3, k + 1, j, i, own));
+    c2p_core<T, false, false, false>(a, g.at(k, j, i), uv, bx, by, bz, false, mdt, nb);
+    return;
+  }
+  if (!v.at(tile - ngt, k, j, i)) return;
+  k += g.ks; j += g.js; i += g.is;
+  const long long c = g.at(k, j, i), cs = g.cstride;
+  const long long cx = i == g.ie && a.bc[0] == 0 ? c + 1 - g.nx1 : c + 1;
+  const double bx = 0.5 * (a.b1[c] + a.b1[cx]);
+  double by = a.b2[c], bz = a.b3[c];
+  if (g.two_d) by = 0.5 * (by + a.b2[j == g.je && a.bc[1] == 0 ? c + (long long)(1 - g.nx2) * g.pitch : c + g.pitch]);
+  if (g.three_d) bz = 0.5 * (bz + a.b3[k == g.ke && a.bc[2] == 0 ? c + (1 - g.nx3) * g.plane : c + g.plane]);
+  const double *u = a.u + c;
+  const double uv[5] = {u[IDN * cs], u[IM1 * cs], u[IM2 * cs], u[IM3 * cs], u[IEN * cs]};
+  c2p_core<T, DT, false, false>(a, c, uv, bx, by, bz, true, mdt, nb);
 }
 
 // The deferred resynchronisation of u[IENT] = rho p / rho^gamma over every cell, with the
@@ -838,17 +757,36 @@ __device__ __forceinline__ void c2p_block_merge(const C2pArgsT<T> &a, double mdt
 // firing stage 13% slower (749 vs 660 us: blocks of four or five tiles leave a long tail), and
 // in the benchmark stage 1 fires every step. One tile per block also keeps the loop-invariant
 // constants of pow() out of the registers of the whole kernel.
-template <class T, bool DT, bool ENT, bool DE>
+// k_c2p: u[IENT] is transported or stored, ghosts filled by a launch before (k_fill).
+// k_fill_c2p: the fast path, with the ghost fill in the same launch. A dependent launch costs about
+// 4.5 us on the device even when it does nothing, and the x1 fill alone touches two lines per row
+// and array for three values (23 us at 192^3); behind the active tiles both are hidden. Against a
+// launch per direction and then con2prim over all cells, ms per pass: 50 steps of 150x129 9.76 ->
+// 8.23, 50 of 512^2 mixed 14.3 -> 12.6, 40 of 64x56x45 16.8 -> 14.7, 20 of 256^3 338 -> 332, 100 of
+// 64 small mixed runs 33.5 -> 30.0. Active rows are also whole lines, which rows with ghosts are not.
+template <class T, bool DT, bool DE>
 __global__ void __launch_bounds__(256) k_c2p(const C2pArgsT<T> a, const VB v) {
   if (!gate(a.ctrl, a.only_if_bad)) return;
   double mdt = 1e300;
   int nbad_local = 0;
   int k, j, i;
-  if (v.at(xcd_tile(int(blockIdx.x), int(gridDim.x), a.xg), k, j, i)) c2p_at<T, DT, ENT, DE>(a, k, j, i, mdt, nbad_local);
+  if (v.at(xcd_tile(int(blockIdx.x), int(gridDim.x), a.xg), k, j, i)) c2p_at<T, DT, true, DE>(a, k, j, i, mdt, nbad_local);
   if (!DT && a.flag_mode != 1) return;
   __shared__ double smin[BX * BY / 64];
   __shared__ int ssum[BX * BY / 64];
   c2p_block_merge<DT>(a, mdt, nbad_local, smin, ssum);
+}
+
+template <class T, bool DT>
+__global__ void __launch_bounds__(256) k_fill_c2p(const C2pArgsT<T> a, const VB v, const int ngt) {
+  if (!gate(a.ctrl, a.only_if_bad)) return;
+  double mdt = 1e300;
+  const int b = int(blockIdx.x);
+  fill_c2p_tile<T, DT>(a, v, b < ngt ? b : ngt + xcd_tile(b - ngt, v.n, a.xg), ngt, mdt);
+  if (!DT || b < ngt) return;
+  __shared__ double smin[BX * BY / 64];
+  __shared__ int ssum[BX * BY / 64];
+  c2p_block_merge<DT>(a, mdt, 0, smin, ssum);
 }
 
 // standalone FlagBadCells over the active cells (fofc.hpp:17-44); count into ctrl->nbad, with
@@ -987,32 +925,18 @@ __global__ void __launch_bounds__(256) kb_update(const RunArgs<T> *R, const Item
   }
 }
 
-template <class T, int DIR>
-__global__ void __launch_bounds__(256) kb_bc(const RunArgs<T> *R, const ItemList L, int buf) {
-  const int n = *L.n;
-  for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[it];
-    if (!R[m.run].ctrl->active) continue;
-    const BcArgs a = R[m.run].bc[buf][DIR];
-    bc_at<DIR>(a, (long long)m.tile * 256 + threadIdx.x);
-  }
-}
-
-// one con2prim tile of a run (the block's CFL minimum and flags merge into that run's
+// one ghost fill / con2prim tile of a run (the block's CFL minimum and flags merge into that run's
 // control block); `cond` selects the fofc re-run (no flags, second minimum slot)
 template <class T, bool LAST>
 __device__ __forceinline__ void c2p_tile(const RunArgs<T> &run, const Ctrl *ctl, int tile, int buf, bool cond,
                                          double *smin, int *ssum) {
   C2pArgsT<T> a = run.c2p[buf][ctl->wcur ^ 1];
   a.compute_dt = LAST;
-  a.entropy_out = 0;   // u[IENT]: deferred to the first host read (k_ient_sync)
   a.slot = cond ? 1 : 0;
   if (cond) a.flag_mode = 0;
   double mdt = 1e300;
-  int nb = 0;
-  int k, j, i;
-  if (c2p_vb(a.g).at(tile, k, j, i)) c2p_at<T, LAST, false, false>(a, k, j, i, mdt, nb);   // batches: no dual energy
-  if (LAST) c2p_block_merge<LAST>(a, mdt, nb, smin, ssum);
+  fill_c2p_tile<T, LAST>(a, active_vb(a.g), tile, ghost_tiles(a.g), mdt);   // batches: no dual energy
+  if (LAST) c2p_block_merge<LAST>(a, mdt, 0, smin, ssum);
 }
 
 template <class T, bool LAST>
@@ -1052,10 +976,7 @@ __global__ void __launch_bounds__(1024) kb_fofc_scan(const RunArgs<T> *R, const 
         cnt[1 + CL_REPAIR] = div_up(nb * 2 * R[r].ndir, 256);
         cnt[1 + CL_CORNER] = div_up(nb * 8, 256);
         cnt[1 + CL_UPDATE] = R[r].cond_tiles[0];
-        cnt[1 + CL_BC1] = R[r].cond_tiles[1];
-        cnt[1 + CL_BC2] = R[r].cond_tiles[2];
-        cnt[1 + CL_BC3] = R[r].cond_tiles[3];
-        cnt[1 + CL_C2P] = R[r].cond_tiles[4];
+        cnt[1 + CL_C2P] = R[r].cond_tiles[1];
       }
     }
     // inclusive wave scans, then the wave offsets
@@ -1128,14 +1049,6 @@ __global__ void __launch_bounds__(256) kb_update_cond(const RunArgs<T> *R, const
   cond_walk(C, CL_UPDATE, [&](int r, int tile) { update_tile(R[r], R[r].ctrl, tile, out, g0, g1, beta); });
 }
 
-template <class T, int DIR>
-__global__ void __launch_bounds__(256) kb_bc_cond(const RunArgs<T> *R, const CondList C, int buf) {
-  cond_walk(C, CL_BC1 + DIR, [&](int r, int tile) {
-    const BcArgs a = R[r].bc[buf][DIR];
-    bc_at<DIR>(a, (long long)tile * 256 + threadIdx.x);
-  });
-}
-
 template <class T, bool LAST>
 __global__ void __launch_bounds__(256) kb_c2p_cond(const RunArgs<T> *R, const CondList C, int buf) {
   __shared__ double smin[BX * BY / 64];
@@ -1145,7 +1058,7 @@ __global__ void __launch_bounds__(256) kb_c2p_cond(const RunArgs<T> *R, const Co
 
 // The rest of the fofc branch of a batch of small runs, after kb_repair_runs: one block per
 // run walks the tiles of its run phase by phase (edge EMFs around the listed cells, the
-// whole-run re-update, boundaries x1 -> x2 -> x3, con2prim), with block barriers between the
+// whole-run re-update, ghost fill and con2prim), with block barriers between the
 // phases; a run that flagged nothing exits at once. The tile bodies are those of the
 // multi-launch branch, so every value is the same.
 template <class T, bool LAST>
@@ -1166,13 +1079,7 @@ __global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *R, const i
   __syncthreads();
   for (int tile = 0; tile < run.cond_tiles[0]; ++tile) update_tile(run, ctl, tile, out, g0, g1, beta);
   __syncthreads();
-  for (int tile = 0; tile < run.cond_tiles[1]; ++tile) bc_at<0>(run.bc[out][0], (long long)tile * 256 + threadIdx.x);
-  __syncthreads();
-  for (int tile = 0; tile < run.cond_tiles[2]; ++tile) bc_at<1>(run.bc[out][1], (long long)tile * 256 + threadIdx.x);
-  __syncthreads();
-  for (int tile = 0; tile < run.cond_tiles[3]; ++tile) bc_at<2>(run.bc[out][2], (long long)tile * 256 + threadIdx.x);
-  __syncthreads();
-  for (int tile = 0; tile < run.cond_tiles[4]; ++tile) c2p_tile<T, LAST>(run, ctl, tile, out, true, smin, ssum);
+  for (int tile = 0; tile < run.cond_tiles[1]; ++tile) c2p_tile<T, LAST>(run, ctl, tile, out, true, smin, ssum);
 }
 
 // live[r] (end of step) = 1 while run r has not reached tlim / nlim
@@ -1263,28 +1170,30 @@ hipError_t launch_update_near(const UpdateArgsT<T> &a, const int *marks, hipStre
 template hipError_t launch_update_near<double>(const UpdateArgsT<double> &, const int *, hipStream_t);
 template hipError_t launch_update_near<float>(const UpdateArgsT<float> &, const int *, hipStream_t);
 
-hipError_t launch_bc(const BcArgs &a, int dir, hipStream_t s) {
-  const int nb = int((bc_points(a.g, dir) + 255) / 256);
-  if (dir == 0) hipLaunchKernelGGL(k_bc<0>, dim3(nb), dim3(256), 0, s, a);
-  else if (dir == 1) hipLaunchKernelGGL(k_bc<1>, dim3(nb), dim3(256), 0, s, a);
-  else hipLaunchKernelGGL(k_bc<2>, dim3(nb), dim3(256), 0, s, a);
+hipError_t launch_fill(const BcArgs &a, hipStream_t s) {
+  hipLaunchKernelGGL(k_fill, dim3(div_up(ghost_points(a.g), 256)), dim3(256), 0, s, a);
   return hipGetLastError();
 }
+
+template <class T>
+hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s) {
+  const VB v = active_vb(a.g);
+  const int ngt = (ghost_tiles(a.g) + 7) & ~7;   // the active tiles start on the first XCD
+  if (a.compute_dt) hipLaunchKernelGGL((k_fill_c2p<T, true>), dim3(ngt + v.n), dim3(256), 0, s, a, v, ngt);
+  else hipLaunchKernelGGL((k_fill_c2p<T, false>), dim3(ngt + v.n), dim3(256), 0, s, a, v, ngt);
+  return hipGetLastError();
+}
+template hipError_t launch_fill_c2p<double>(const C2pArgsT<double> &, hipStream_t);
+template hipError_t launch_fill_c2p<float>(const C2pArgsT<float> &, hipStream_t);
 
 namespace {
 template <class T, bool DE>
 void launch_c2p_de(const C2pArgsT<T> &a, hipStream_t s) {
   const Geom &g = a.g;
-  const bool ent = a.entropy_out || a.eos.dual_energy;
   const VB v = c2p_vb(g);
   const dim3 grid(v.n), block(256);
-  if (a.compute_dt) {
-    if (ent) hipLaunchKernelGGL((k_c2p<T, true, true, DE>), grid, block, 0, s, a, v);
-    else hipLaunchKernelGGL((k_c2p<T, true, false, DE>), grid, block, 0, s, a, v);
-  } else {
-    if (ent) hipLaunchKernelGGL((k_c2p<T, false, true, DE>), grid, block, 0, s, a, v);
-    else hipLaunchKernelGGL((k_c2p<T, false, false, DE>), grid, block, 0, s, a, v);
-  }
+  if (a.compute_dt) hipLaunchKernelGGL((k_c2p<T, true, DE>), grid, block, 0, s, a, v);
+  else hipLaunchKernelGGL((k_c2p<T, false, DE>), grid, block, 0, s, a, v);
 }
 }  // namespace
 
@@ -1348,13 +1257,6 @@ hipError_t launchb_update(const RunArgs<T> *R, ItemList L, int out, double g0, d
   return hipGetLastError();
 }
 template <class T>
-hipError_t launchb_bc(const RunArgs<T> *R, ItemList L, int dir, int buf, int grid, hipStream_t s) {
-  if (dir == 0) hipLaunchKernelGGL((kb_bc<T, 0>), dim3(grid), dim3(256), 0, s, R, L, buf);
-  else if (dir == 1) hipLaunchKernelGGL((kb_bc<T, 1>), dim3(grid), dim3(256), 0, s, R, L, buf);
-  else hipLaunchKernelGGL((kb_bc<T, 2>), dim3(grid), dim3(256), 0, s, R, L, buf);
-  return hipGetLastError();
-}
-template <class T>
 hipError_t launchb_c2p(const RunArgs<T> *R, ItemList L, int buf, int last, int grid, hipStream_t s) {
   if (last) hipLaunchKernelGGL((kb_c2p<T, true>), dim3(grid), dim3(256), 0, s, R, L, buf);
   else hipLaunchKernelGGL((kb_c2p<T, false>), dim3(grid), dim3(256), 0, s, R, L, buf);
@@ -1374,13 +1276,6 @@ template <class T>
 hipError_t launchb_update_cond(const RunArgs<T> *R, CondList C, int out, double g0, double g1, double beta, int grid,
                                hipStream_t s) {
   hipLaunchKernelGGL(kb_update_cond<T>, dim3(grid), dim3(256), 0, s, R, C, out, g0, g1, beta);
-  return hipGetLastError();
-}
-template <class T>
-hipError_t launchb_bc_cond(const RunArgs<T> *R, CondList C, int dir, int buf, int grid, hipStream_t s) {
-  if (dir == 0) hipLaunchKernelGGL((kb_bc_cond<T, 0>), dim3(grid), dim3(256), 0, s, R, C, buf);
-  else if (dir == 1) hipLaunchKernelGGL((kb_bc_cond<T, 1>), dim3(grid), dim3(256), 0, s, R, C, buf);
-  else hipLaunchKernelGGL((kb_bc_cond<T, 2>), dim3(grid), dim3(256), 0, s, R, C, buf);
   return hipGetLastError();
 }
 template <class T>
@@ -1408,13 +1303,11 @@ hipError_t launchb_ctrl(const RunArgs<T> *R, const int *nruns, int cap, int op, 
   template hipError_t launchb_corner<T>(const RunArgs<T> *, ItemList, int, hipStream_t);                     \
   template hipError_t launchb_update<T>(const RunArgs<T> *, ItemList, int, double, double, double, int,      \
                                         hipStream_t);                                                         \
-  template hipError_t launchb_bc<T>(const RunArgs<T> *, ItemList, int, int, int, hipStream_t);               \
   template hipError_t launchb_c2p<T>(const RunArgs<T> *, ItemList, int, int, int, hipStream_t);              \
   template hipError_t launchb_fofc_scan<T>(const RunArgs<T> *, const int *, CondList, hipStream_t);          \
   template hipError_t launchb_corner_cond<T>(const RunArgs<T> *, CondList, int, hipStream_t);                \
   template hipError_t launchb_update_cond<T>(const RunArgs<T> *, CondList, int, double, double, double, int, \
                                              hipStream_t);                                                    \
-  template hipError_t launchb_bc_cond<T>(const RunArgs<T> *, CondList, int, int, int, hipStream_t);          \
   template hipError_t launchb_c2p_cond<T>(const RunArgs<T> *, CondList, int, int, int, hipStream_t);         \
   template hipError_t launchb_fofc_runs<T>(const RunArgs<T> *, const int *, int, int, double, double, double, int, \
                                            hipStream_t);         \
