@@ -723,7 +723,7 @@ int chq_init_resume(chq_ctx *c, double t, int cycle, double tlim, int nlim) {
 extern "C++" {
 // One fused RK stage (dual energy off) over field set `fs` (FP64, or FP32 in mixed precision).
 template <class T>
-static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf, int last) {
+static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf, int last, const CtrlTurn &turn) {
   const Recon rc = Recon(c->cfg.recon);
   const RSolver rs = RSolver(c->cfg.rsolver);
   Ctrl *k = c->ctrl;
@@ -840,9 +840,13 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
     cb.flag_mode = 0;
     cb.slot = 1;
     cb.only_if_bad = 1;   // (after ca's gate 2: exactly one of the two runs)
-    HIPCHK(c->entropy ? launch_c2p<T>(cb, c->stream) : launch_fill_c2p<T>(cb, c->stream));
+    // the stage's control turn goes with this launch where it can
+    const bool with_turn = !c->entropy && fill_c2p_tiles(c->g) <= FILL_TURN_TILES;
+    HIPCHK(c->entropy ? launch_c2p<T>(cb, c->stream) : launch_fill_c2p<T>(cb, c->stream, with_turn ? &turn : nullptr));
     c->tmark(CHQ_K_REPAIR, false);
+    if (with_turn) return CHQ_OK;
   }
+  HIPCHK(launch_ctrl_turn(c->ctrl, turn, c->stream));
   return CHQ_OK;
 }
 }  // extern "C++"
@@ -855,7 +859,10 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
 // on: without it con2prim recomputes u[IENT] from rho and p in every stage, so its transport
 // cannot change any result. With dual energy or the flux limiter on, the flag runs before the
 // boundary fill (see enqueue_fused_stage); explicit diffusion keeps the reference kernel order.
-static int enqueue_step(chq_ctx *c) {
+// `first` / `more`: the first step of the call / another one follows in it. The control work
+// between two stages is one turn (CtrlTurn), and so is that between two steps of a call unless
+// a split step or the parabolic limit comes between the last stage and the step's end.
+static int enqueue_step(chq_ctx *c, bool first, bool more) {
   const Recon rc = Recon(c->cfg.recon);
   const RSolver rs = RSolver(c->cfg.rsolver);
   Ctrl *k = c->ctrl;
@@ -866,14 +873,28 @@ static int enqueue_step(chq_ctx *c) {
   const bool split = c->cfg.sts || c->cfg.cooling;   // main.cpp:273-290: dt taken after the splits
   const bool fused = !(c->diffusive() && !c->cfg.sts);
   const int nvar = c->entropy ? 6 : 5;
-  HIPCHK(launch_ctrl_begin_step(k, c->stream));
+  const bool tail = split || (!fused && c->diffusive());   // work after the last stage
+  if (first || tail) {
+    CtrlTurn t{};
+    t.begin_step = t.begin_stage = 1;
+    t.reset = nst == 1;
+    HIPCHK(launch_ctrl_turn(k, t, c->stream));
+  }
   for (int s = 1; s <= nst; ++s) {
     const Coef cf = rk_coef(nst, s);
     const int last = s == nst;
-    HIPCHK(launch_ctrl_begin_stage(k, last, c->stream, s - 1));
+    CtrlTurn turn{};
+    turn.end_stage = 1;
+    turn.last = last;
+    turn.fused = fused;
+    turn.end_step = last && !tail;
+    turn.begin_step = last && !tail && more;
+    turn.begin_stage = !last || turn.begin_step;
+    turn.stage = last ? 0 : s;
+    turn.reset = turn.stage == nst - 1;
     if (fused) {
-      const int rc2 = c->mixed ? enqueue_fused_stage<float>(c, c->f32, cf, last)
-                               : enqueue_fused_stage<double>(c, c->f64, cf, last);
+      const int rc2 = c->mixed ? enqueue_fused_stage<float>(c, c->f32, cf, last, turn)
+                               : enqueue_fused_stage<double>(c, c->f64, cf, last, turn);
       if (rc2) return rc2;
       c->wcur ^= 1;
     } else {
@@ -920,8 +941,8 @@ static int enqueue_step(chq_ctx *c) {
       ca.compute_dt = last && !split;   // main.cpp:273-274: split steps take dt after the splits
       ca.slot = 0;
       HIPCHK(launch_c2p<double>(ca, c->stream));
+      HIPCHK(launch_ctrl_turn(k, turn, c->stream));
     }
-    HIPCHK(launch_ctrl_end_stage(k, last, fused ? 1 : 0, c->stream));
     if (last && !fused && !split && c->diffusive()) {   // main.cpp:275
       HIPCHK(launch_rho_min(c->f64.w[c->wcur], c->g, k, true, c->stream));
       HIPCHK(launch_diff_dt_fold(k, c->diff_args(0, c->wcur, k, false), c->stream));
@@ -961,7 +982,11 @@ static int enqueue_step(chq_ctx *c) {
       HIPCHK(launch_diff_dt_fold(k, c->diff_args(0, c->wcur, k, false), c->stream));
     }
   }
-  HIPCHK(launch_ctrl_end_step(k, c->stream));
+  if (tail) {
+    CtrlTurn t{};
+    t.end_step = 1;
+    HIPCHK(launch_ctrl_turn(k, t, c->stream));
+  }
   c->wcur_stale = fused;
   return CHQ_OK;
 }
@@ -971,7 +996,7 @@ int chq_step(chq_ctx *c, int nsteps) {
   if (c->batch) return fail(CHQ_EINVAL, "this context is advanced by a batch");
   if (int rc_ = sync_wcur(c)) return rc_;
   for (int n = 0; n < nsteps; ++n) {
-    const int rc = enqueue_step(c);
+    const int rc = enqueue_step(c, n == 0, n + 1 < nsteps);
     if (rc) return rc;
   }
   return CHQ_OK;

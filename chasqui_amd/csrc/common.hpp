@@ -57,6 +57,7 @@ struct Ctrl {
   int stage;                     // RK stage index of the time loop (-1: a single-kernel entry point)
   int fired;                     // bit s: stage s of the last step flagged cells
   int epoch;                     // stages begun since the loop started (near-marks of the local re-update)
+  int done;                      // blocks of a launch that ends with a control turn (CtrlTurn)
   int zsens;                     // first-pass points the local fofc re-update cannot skip (zero sign, non-finite)
 };
 

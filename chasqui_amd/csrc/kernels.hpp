@@ -375,15 +375,23 @@ hipError_t launch_limit_fluxes(const SrcArgs &a, int dir, hipStream_t s);
 hipError_t launch_gravity(const SrcArgs &a, hipStream_t s);
 hipError_t launch_cooling(const SrcArgs &a, hipStream_t s);
 template <class T> hipError_t launch_c2p(const C2pArgsT<T> &a, hipStream_t s);
-// ghost fill and con2prim of every cell in one launch (u[IENT] neither transported nor stored)
-template <class T> hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s);
+// The control work between two stages, in this order: end of a stage (`last` of its step), end
+// of the step, begin of the next step, begin of a stage (`stage`, `reset` the CFL minima). One
+// launch, or none where a conditional con2prim launch takes it along (launch_fill_c2p).
+struct CtrlTurn {
+  int end_stage, last, fused, end_step, begin_step, begin_stage, reset, stage;
+};
+hipError_t launch_ctrl_turn(Ctrl *c, const CtrlTurn &t, hipStream_t s);
+// ghost fill and con2prim of every cell in one launch (u[IENT] neither transported nor stored).
+// With `turn` (a launch whose gate is closed by nbad == 0, at most FILL_TURN_TILES tiles), the
+// launch ends with that control turn.
+constexpr int FILL_TURN_TILES = 2048;
+inline int fill_c2p_tiles(const Geom &g) { return ((ghost_tiles(g) + 7) & ~7) + active_vb(g).n; }
+template <class T> hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s, const CtrlTurn *turn = nullptr);
 hipError_t launch_flag(const C2pArgs &a, hipStream_t s);   // standalone FlagBadCells
 // control-block kernels
-hipError_t launch_ctrl_begin_step(Ctrl *c, hipStream_t s);
-// stage: RK stage index of the time loop (selects the adaptive fofc order), -1 otherwise
-hipError_t launch_ctrl_begin_stage(Ctrl *c, int reset_slots, hipStream_t s, int stage = -1);
-hipError_t launch_ctrl_end_stage(Ctrl *c, int last, int fused, hipStream_t s);
-hipError_t launch_ctrl_end_step(Ctrl *c, hipStream_t s);
+// outside the time loop (the per-kernel entry points and split steps)
+hipError_t launch_ctrl_begin_stage(Ctrl *c, int reset_slots, hipStream_t s);
 
 // batched launches: `grid` blocks walk the list (grid-stride); stage coefficients are
 // launch arguments, everything per run comes from the RunArgs table

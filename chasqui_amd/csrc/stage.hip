@@ -749,6 +749,63 @@ __device__ __forceinline__ void c2p_block_merge(const C2pArgsT<T> &a, double mdt
   __syncthreads();   // smin / ssum are reused by the next tile of a grid-stride loop
 }
 
+// ---------------------------------------------------------------- control
+__device__ __forceinline__ unsigned long long bits_of(double x) { return (unsigned long long)__double_as_longlong(x); }
+__device__ __forceinline__ double from_bits(unsigned long long b) { return __longlong_as_double((long long)b); }
+
+// main.cpp:243-248 (nlim counts the cycles run since the loop started, main.cpp:243)
+__device__ __forceinline__ bool ctrl_running(const Ctrl *c) {
+  return c->t < c->tlim && (c->nlim < 0 || c->cycle - c->cycle0 < c->nlim);
+}
+__device__ __forceinline__ void ctrl_begin_step(Ctrl *c) {
+  if (!ctrl_running(c)) { c->active = 0; return; }
+  c->active = 1;
+  double dt = c->cfl * c->min_dt;
+  if (c->t + dt > c->tlim) dt = c->tlim - c->t;
+  c->dt = dt;
+}
+// The adaptive fofc order: an RK stage whose counterpart in the previous step flagged cells
+// flags right after the update, before the boundary fill (the reference's order), so when it
+// fires again it fills and converts once; other stages keep the flag inside con2prim and pay a
+// second fill and con2prim only when they fire. Firing clusters by stage (the first stage's
+// full forward step, mostly), not from one stage to the next. Both orders give the same bits:
+// boundaries never change the active cells the flag reads. stage -1 (the single-kernel entry
+// points) never flags early.
+__device__ __forceinline__ void ctrl_begin_stage(Ctrl *c, int reset_slots, int stage) {
+  c->epoch += 1;
+  c->zsens = 0;
+  c->stage = stage;
+  c->early = stage >= 0 && ((c->fired >> stage) & 1);
+  c->nbad = 0;
+  if (reset_slots) { c->mdt_bits[0] = bits_of(1e300); c->mdt_bits[1] = bits_of(1e300); }
+}
+// the CFL minimum of the final (possibly fofc-repaired) con2prim of the last stage
+// (fused order: slot 1 holds the minimum of the repaired state when cells were flagged).
+// The fused order alternates the primitive sets every stage that ran.
+__device__ __forceinline__ void ctrl_end_stage(Ctrl *c, int last, int fused) {
+  if (!c->active) return;
+  if (fused) c->wcur ^= 1;
+  c->fofc_total += c->nbad;
+  c->nbad_last = c->nbad;
+  if (c->stage >= 0) c->fired = c->nbad ? (c->fired | (1 << c->stage)) : (c->fired & ~(1 << c->stage));
+  // (an atomic load: the turn at the end of a con2prim launch follows other blocks' atomics)
+  if (last)
+    c->min_dt = fmin(from_bits(__hip_atomic_load(&c->mdt_bits[(fused && c->nbad) ? 1 : 0], __ATOMIC_RELAXED,
+                                                 __HIP_MEMORY_SCOPE_AGENT)), 1e300);
+}
+// main.cpp:291-292
+__device__ __forceinline__ void ctrl_end_step(Ctrl *c) {
+  if (!c->active) return;
+  c->t += c->dt;
+  c->cycle += 1;
+}
+__device__ __forceinline__ void ctrl_turn(Ctrl *c, const CtrlTurn &t) {
+  if (t.end_stage) ctrl_end_stage(c, t.last, t.fused);
+  if (t.end_step) ctrl_end_step(c);
+  if (t.begin_step) ctrl_begin_step(c);
+  if (t.begin_stage) ctrl_begin_stage(c, t.reset, t.stage);
+}
+
 // cons -> prim over all cells, physics.hpp:437-494. The CFL minimum is reduced with wave64
 // shuffles and one LDS pass per block, then merged with a 64-bit atomicMin on the bit
 // pattern, issued only when the block's minimum beats the current one.
@@ -777,16 +834,36 @@ __global__ void __launch_bounds__(256) k_c2p(const C2pArgsT<T> a, const VB v) {
   c2p_block_merge<DT>(a, mdt, nbad_local, smin, ssum);
 }
 
-template <class T, bool DT>
-__global__ void __launch_bounds__(256) k_fill_c2p(const C2pArgsT<T> a, const VB v, const int ngt) {
-  if (!gate(a.ctrl, a.only_if_bad)) return;
+// TURN: the fofc-branch re-run (gate 1), which ends the stage with the control turn `t`. With the
+// gate closed (nothing flagged, or the run has ended) the first block does it at once: no block
+// has work, and the turn leaves the gate closed for the others (nbad 0, `active` never set
+// again). With the gate open the last block to finish does it, counted in Ctrl::done after the
+// block's own CFL minimum has arrived (the wait); one counter limits that to FILL_TURN_TILES
+// tiles. With one turn in place of two to four control launches, ms per pass: 100 steps of a 1D
+// run of 128 cells 13.2 -> 11.3, 50 of 150x129 8.23 -> 7.79, 40 of 64x56x45 14.7 -> 14.4.
+template <class T, bool DT, bool TURN>
+__global__ void __launch_bounds__(256) k_fill_c2p(const C2pArgsT<T> a, const VB v, const int ngt, const CtrlTurn t) {
+  if (!gate(a.ctrl, a.only_if_bad)) {
+    if (TURN && blockIdx.x == 0 && threadIdx.x == 0) ctrl_turn(a.ctrl, t);
+    return;
+  }
   double mdt = 1e300;
   const int b = int(blockIdx.x);
   fill_c2p_tile<T, DT>(a, v, b < ngt ? b : ngt + xcd_tile(b - ngt, v.n, a.xg), ngt, mdt);
-  if (!DT || b < ngt) return;
-  __shared__ double smin[BX * BY / 64];
-  __shared__ int ssum[BX * BY / 64];
-  c2p_block_merge<DT>(a, mdt, 0, smin, ssum);
+  if (DT && b >= ngt) {
+    __shared__ double smin[BX * BY / 64];
+    __shared__ int ssum[BX * BY / 64];
+    c2p_block_merge<DT>(a, mdt, 0, smin, ssum);
+  }
+  if constexpr (TURN) {
+    if (threadIdx.x == 0) {
+      __builtin_amdgcn_s_waitcnt(0);   // this thread's atomicMin is done
+      if (__hip_atomic_fetch_add(&a.ctrl->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == int(gridDim.x) - 1) {
+        a.ctrl->done = 0;
+        ctrl_turn(a.ctrl, t);
+      }
+    }
+  }
 }
 
 // standalone FlagBadCells over the active cells (fofc.hpp:17-44); count into ctrl->nbad, with
@@ -827,57 +904,9 @@ __global__ void __launch_bounds__(BX * BY) k_flag(const C2pArgs a) {
   if ((int(threadIdx.x) & 63) == 0 && ws) atomicAdd(&a.ctrl->nbad, ws);
 }
 
-// ---------------------------------------------------------------- control
-__device__ __forceinline__ unsigned long long bits_of(double x) { return (unsigned long long)__double_as_longlong(x); }
-__device__ __forceinline__ double from_bits(unsigned long long b) { return __longlong_as_double((long long)b); }
-
-// main.cpp:243-248 (nlim counts the cycles run since the loop started, main.cpp:243)
-__device__ __forceinline__ bool ctrl_running(const Ctrl *c) {
-  return c->t < c->tlim && (c->nlim < 0 || c->cycle - c->cycle0 < c->nlim);
-}
-__device__ __forceinline__ void ctrl_begin_step(Ctrl *c) {
-  if (!ctrl_running(c)) { c->active = 0; return; }
-  c->active = 1;
-  double dt = c->cfl * c->min_dt;
-  if (c->t + dt > c->tlim) dt = c->tlim - c->t;
-  c->dt = dt;
-}
-// The adaptive fofc order: an RK stage whose counterpart in the previous step flagged cells
-// flags right after the update, before the boundary fill (the reference's order), so when it
-// fires again it fills and converts once; other stages keep the flag inside con2prim and pay a
-// second fill and con2prim only when they fire. Firing clusters by stage (the first stage's
-// full forward step, mostly), not from one stage to the next. Both orders give the same bits:
-// boundaries never change the active cells the flag reads. stage -1 (the single-kernel entry
-// points) never flags early.
-__device__ __forceinline__ void ctrl_begin_stage(Ctrl *c, int reset_slots, int stage) {
-  c->epoch += 1;
-  c->zsens = 0;
-  c->stage = stage;
-  c->early = stage >= 0 && ((c->fired >> stage) & 1);
-  c->nbad = 0;
-  if (reset_slots) { c->mdt_bits[0] = bits_of(1e300); c->mdt_bits[1] = bits_of(1e300); }
-}
-// the CFL minimum of the final (possibly fofc-repaired) con2prim of the last stage
-// (fused order: slot 1 holds the minimum of the repaired state when cells were flagged).
-// The fused order alternates the primitive sets every stage that ran.
-__device__ __forceinline__ void ctrl_end_stage(Ctrl *c, int last, int fused) {
-  if (!c->active) return;
-  if (fused) c->wcur ^= 1;
-  c->fofc_total += c->nbad;
-  c->nbad_last = c->nbad;
-  if (c->stage >= 0) c->fired = c->nbad ? (c->fired | (1 << c->stage)) : (c->fired & ~(1 << c->stage));
-  if (last) c->min_dt = fmin(from_bits(c->mdt_bits[(fused && c->nbad) ? 1 : 0]), 1e300);
-}
-// main.cpp:291-292
-__device__ __forceinline__ void ctrl_end_step(Ctrl *c) {
-  if (!c->active) return;
-  c->t += c->dt;
-  c->cycle += 1;
-}
-__global__ void k_begin_step(Ctrl *c) { ctrl_begin_step(c); }
-__global__ void k_begin_stage(Ctrl *c, int reset_slots, int stage) { ctrl_begin_stage(c, reset_slots, stage); }
-__global__ void k_end_stage(Ctrl *c, int last, int fused) { ctrl_end_stage(c, last, fused); }
-__global__ void k_end_step(Ctrl *c) { ctrl_end_step(c); }
+// ---------------------------------------------------------------- control kernels
+__global__ void k_begin_stage(Ctrl *c, int reset_slots) { ctrl_begin_stage(c, reset_slots, -1); }
+__global__ void k_ctrl_turn(Ctrl *c, const CtrlTurn t) { ctrl_turn(c, t); }
 
 // ---------------------------------------------------------------- batched kernels
 // Grid-stride walks over device-resident (run, tile) lists; each item runs the same tile body
@@ -1176,15 +1205,23 @@ hipError_t launch_fill(const BcArgs &a, hipStream_t s) {
 }
 
 template <class T>
-hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s) {
+hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s, const CtrlTurn *turn) {
   const VB v = active_vb(a.g);
   const int ngt = (ghost_tiles(a.g) + 7) & ~7;   // the active tiles start on the first XCD
-  if (a.compute_dt) hipLaunchKernelGGL((k_fill_c2p<T, true>), dim3(ngt + v.n), dim3(256), 0, s, a, v, ngt);
-  else hipLaunchKernelGGL((k_fill_c2p<T, false>), dim3(ngt + v.n), dim3(256), 0, s, a, v, ngt);
+  const dim3 grid(ngt + v.n), block(256);
+  const CtrlTurn t = turn ? *turn : CtrlTurn{};
+  if (turn && (a.only_if_bad != 1 || int(grid.x) > FILL_TURN_TILES)) return hipErrorInvalidValue;
+  if (a.compute_dt) {
+    if (turn) hipLaunchKernelGGL((k_fill_c2p<T, true, true>), grid, block, 0, s, a, v, ngt, t);
+    else hipLaunchKernelGGL((k_fill_c2p<T, true, false>), grid, block, 0, s, a, v, ngt, t);
+  } else {
+    if (turn) hipLaunchKernelGGL((k_fill_c2p<T, false, true>), grid, block, 0, s, a, v, ngt, t);
+    else hipLaunchKernelGGL((k_fill_c2p<T, false, false>), grid, block, 0, s, a, v, ngt, t);
+  }
   return hipGetLastError();
 }
-template hipError_t launch_fill_c2p<double>(const C2pArgsT<double> &, hipStream_t);
-template hipError_t launch_fill_c2p<float>(const C2pArgsT<float> &, hipStream_t);
+template hipError_t launch_fill_c2p<double>(const C2pArgsT<double> &, hipStream_t, const CtrlTurn *);
+template hipError_t launch_fill_c2p<float>(const C2pArgsT<float> &, hipStream_t, const CtrlTurn *);
 
 namespace {
 template <class T, bool DE>
@@ -1227,20 +1264,12 @@ hipError_t launch_flag(const C2pArgs &a, hipStream_t s) {
   return hipGetLastError();
 }
 
-hipError_t launch_ctrl_begin_step(Ctrl *c, hipStream_t s) {
-  hipLaunchKernelGGL(k_begin_step, dim3(1), dim3(1), 0, s, c);
+hipError_t launch_ctrl_begin_stage(Ctrl *c, int reset_slots, hipStream_t s) {
+  hipLaunchKernelGGL(k_begin_stage, dim3(1), dim3(1), 0, s, c, reset_slots);
   return hipGetLastError();
 }
-hipError_t launch_ctrl_begin_stage(Ctrl *c, int reset_slots, hipStream_t s, int stage) {
-  hipLaunchKernelGGL(k_begin_stage, dim3(1), dim3(1), 0, s, c, reset_slots, stage);
-  return hipGetLastError();
-}
-hipError_t launch_ctrl_end_stage(Ctrl *c, int last, int fused, hipStream_t s) {
-  hipLaunchKernelGGL(k_end_stage, dim3(1), dim3(1), 0, s, c, last, fused);
-  return hipGetLastError();
-}
-hipError_t launch_ctrl_end_step(Ctrl *c, hipStream_t s) {
-  hipLaunchKernelGGL(k_end_step, dim3(1), dim3(1), 0, s, c);
+hipError_t launch_ctrl_turn(Ctrl *c, const CtrlTurn &t, hipStream_t s) {
+  hipLaunchKernelGGL(k_ctrl_turn, dim3(1), dim3(1), 0, s, c, t);
   return hipGetLastError();
 }
 
