@@ -466,13 +466,14 @@ hipError_t launch_repair_list_t(const FluxArgsT<T> a[3], int ndir, const int *li
 // Grid-stride walks over (run, tile) lists of a batch; the tile bodies are the ones above,
 // with the run's launch description for its current primitive set (Ctrl::wcur).
 template <class T, Recon RC, RSolver RS>
-__global__ void __launch_bounds__(256) kb_flux_x(const RunArgs<T> *R, const ItemList L, const int cur) {
-  const int n = *L.n;
+__global__ void __launch_bounds__(256) kb_flux_x(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+                                                 const int *__restrict__ nitem, const int cur) {
+  const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[it];
+    const Item m = uniform_item(item, it);
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
-    const FluxArgsT<T> a = R[m.run].flux[cur][ctl->wcur][0];
+    const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][0];
     int nseg, nwaves;
     x_shape(a, fpw_v<RC>, nseg, nwaves);
     const int wave = m.tile * 4 + int(threadIdx.x >> 6);
@@ -481,13 +482,14 @@ __global__ void __launch_bounds__(256) kb_flux_x(const RunArgs<T> *R, const Item
 }
 
 template <class T, int DIR, Recon RC, RSolver RS>
-__global__ void __launch_bounds__(BX * BY) kb_flux_m(const RunArgs<T> *R, const ItemList L, const int cur) {
-  const int n = *L.n;
+__global__ void __launch_bounds__(BX * BY) kb_flux_m(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+                                                 const int *__restrict__ nitem, const int cur) {
+  const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[it];
+    const Item m = uniform_item(item, it);
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
-    const FluxArgsT<T> a = R[m.run].flux[cur][ctl->wcur][DIR];
+    const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][DIR];
     flux_m_tile<T, DIR, RC, RS, false>(a, m.tile);
   }
 }
@@ -498,7 +500,7 @@ template <class T>
 __device__ __forceinline__ void repair_entry(const RunArgs<T> &run, const Ctrl *ctl, int t, int cur) {
   const int per = 2 * run.ndir;
   if (t >= ctl->nbad * per) return;
-  const FluxArgsT<T> *fa = run.flux[cur][ctl->wcur];
+  const FluxArgsT<T> *fa = run.flux[cur][uniform(ctl->wcur)];
   const Geom &g = fa[0].g;
   const long long c0 = run.badlist[t / per];
   const int q = t % per, dir = q >> 1, side = q & 1;
@@ -508,7 +510,7 @@ __device__ __forceinline__ void repair_entry(const RunArgs<T> &run, const Ctrl *
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) kb_repair(const RunArgs<T> *R, const CondList C, const int cur) {
+__global__ void __launch_bounds__(256) kb_repair(const RunArgs<T> *__restrict__ R, const CondList C, const int cur) {
   const int nrun = *C.nrun();
   if (nrun == 0) return;
   const int *pre = C.pre(CL_REPAIR);
@@ -523,7 +525,7 @@ __global__ void __launch_bounds__(256) kb_repair(const RunArgs<T> *R, const Cond
 // The repair of a batch of small runs: one block per run, which walks its run's entries
 // (runs that flagged nothing exit at once; no compaction pass is needed).
 template <class T>
-__global__ void __launch_bounds__(256) kb_repair_runs(const RunArgs<T> *R, const int *nruns, const int cur) {
+__global__ void __launch_bounds__(256) kb_repair_runs(const RunArgs<T> *__restrict__ R, const int *nruns, const int cur) {
   const int r = int(blockIdx.x);
   if (r >= *nruns) return;
   const Ctrl *ctl = R[r].ctrl;
@@ -535,14 +537,14 @@ __global__ void __launch_bounds__(256) kb_repair_runs(const RunArgs<T> *R, const
 template <class T, int DIR, Recon RC>
 hipError_t gob_flux_rs(const RunArgs<T> *R, ItemList L, int cur, RSolver rs, int grid, hipStream_t s) {
   if constexpr (DIR == 0) {
-    if (rs == RSolver::hlld) hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::hlld>), dim3(grid), dim3(256), 0, s, R, L, cur);
-    else if (rs == RSolver::lhlld) hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::lhlld>), dim3(grid), dim3(256), 0, s, R, L, cur);
-    else hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::hlle>), dim3(grid), dim3(256), 0, s, R, L, cur);
+    if (rs == RSolver::hlld) hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::hlld>), dim3(grid), dim3(256), 0, s, R, L.item, L.n, cur);
+    else if (rs == RSolver::lhlld) hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::lhlld>), dim3(grid), dim3(256), 0, s, R, L.item, L.n, cur);
+    else hipLaunchKernelGGL((kb_flux_x<T, RC, RSolver::hlle>), dim3(grid), dim3(256), 0, s, R, L.item, L.n, cur);
   } else {
     const dim3 b(BX, BY, 1);
-    if (rs == RSolver::hlld) hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::hlld>), dim3(grid), b, 0, s, R, L, cur);
-    else if (rs == RSolver::lhlld) hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::lhlld>), dim3(grid), b, 0, s, R, L, cur);
-    else hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::hlle>), dim3(grid), b, 0, s, R, L, cur);
+    if (rs == RSolver::hlld) hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::hlld>), dim3(grid), b, 0, s, R, L.item, L.n, cur);
+    else if (rs == RSolver::lhlld) hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::lhlld>), dim3(grid), b, 0, s, R, L.item, L.n, cur);
+    else hipLaunchKernelGGL((kb_flux_m<T, DIR, RC, RSolver::hlle>), dim3(grid), b, 0, s, R, L.item, L.n, cur);
   }
   return hipGetLastError();
 }

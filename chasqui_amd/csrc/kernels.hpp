@@ -420,6 +420,16 @@ template <class T> hipError_t launchb_ctrl(const RunArgs<T> *R, const int *nruns
 enum : int { CTRL_BEGIN_STEP = 0, CTRL_BEGIN_STAGE, CTRL_END_STAGE, CTRL_END_STEP, CTRL_LIVE, CTRL_STEP_FIRST,
              CTRL_TURN, CTRL_END_LAST };
 
+// A batched kernel's item and its run's launch description are the same for every lane of a wave.
+// Said so (and the tables __restrict__: nothing a kernel writes aliases them), they are read by
+// scalar loads into SGPRs; as vector loads they held 45 to 60 VGPRs of each kernel (con2prim 90-102
+// against 46 in the single-mesh form) and stood in front of every tile's own loads. 48 vortices of
+// 64^2 to 512^2, FP64, 40 steps: 143.2 -> 136.0 ms.
+__device__ __forceinline__ int uniform(int v) { return __builtin_amdgcn_readfirstlane(v); }
+__device__ __forceinline__ Item uniform_item(const Item *__restrict__ item, int it) {
+  return Item{uniform(item[it].run), uniform(item[it].tile)};
+}
+
 // position of `it` in an exclusive prefix pre[0..n] (largest p with pre[p] <= it)
 __device__ __forceinline__ int locate(const int *pre, int n, int it) {
   int lo = 0, hi = n - 1;

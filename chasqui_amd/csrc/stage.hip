@@ -914,13 +914,14 @@ __global__ void k_ctrl_turn(Ctrl *c, const CtrlTurn t) { ctrl_turn(c, t); }
 // The primitive set a run reads is its Ctrl::wcur; con2prim writes the other one.
 
 template <class T>
-__global__ void __launch_bounds__(256) kb_corner(const RunArgs<T> *R, const ItemList L) {
-  const int n = *L.n;
+__global__ void __launch_bounds__(256) kb_corner(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+                                                 const int *__restrict__ nitem) {
+  const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[xcd_tile(it, n, XG_CORNER)];   // (the grids are multiples of 8 blocks)
+    const Item m = uniform_item(item, xcd_tile(it, n, XG_CORNER));   // (the grids are multiples of 8 blocks)
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
-    const CornerArgsT<T> a = R[m.run].corner[ctl->wcur];
+    const CornerArgsT<T> a = R[m.run].corner[uniform(ctl->wcur)];
     const Geom &g = a.g;
     int k, j, i;
     if (!corner_vb(g).at(m.tile, k, j, i)) continue;
@@ -942,12 +943,13 @@ __device__ __forceinline__ void update_tile(const RunArgs<T> &run, const Ctrl *c
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) kb_update(const RunArgs<T> *R, const ItemList L, int out, double g0, double g1,
+__global__ void __launch_bounds__(256) kb_update(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+                                                 const int *__restrict__ nitem, int out, double g0, double g1,
                                                  double beta) {
-  const int n = *L.n;
+  const int n = *nitem;
   const int grp = std::is_same<T, float>::value ? XG_UPDATE_F32 : 0;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[xcd_tile(it, n, grp)];
+    const Item m = uniform_item(item, xcd_tile(it, n, grp));
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     update_tile(R[m.run], ctl, m.tile, out, g0, g1, beta);
@@ -959,7 +961,7 @@ __global__ void __launch_bounds__(256) kb_update(const RunArgs<T> *R, const Item
 template <class T, bool LAST>
 __device__ __forceinline__ void c2p_tile(const RunArgs<T> &run, const Ctrl *ctl, int tile, int buf, bool cond,
                                          double *smin, int *ssum) {
-  C2pArgsT<T> a = run.c2p[buf][ctl->wcur ^ 1];
+  C2pArgsT<T> a = run.c2p[buf][uniform(ctl->wcur) ^ 1];
   a.compute_dt = LAST;
   a.slot = cond ? 1 : 0;
   if (cond) a.flag_mode = 0;
@@ -969,12 +971,13 @@ __device__ __forceinline__ void c2p_tile(const RunArgs<T> &run, const Ctrl *ctl,
 }
 
 template <class T, bool LAST>
-__global__ void __launch_bounds__(256) kb_c2p(const RunArgs<T> *R, const ItemList L, int buf) {
+__global__ void __launch_bounds__(256) kb_c2p(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+                                                 const int *__restrict__ nitem, int buf) {
   __shared__ double smin[BX * BY / 64];
   __shared__ int ssum[BX * BY / 64];
-  const int n = *L.n;
+  const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = L.item[xcd_tile(it, n, XG_C2P)];
+    const Item m = uniform_item(item, xcd_tile(it, n, XG_C2P));
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     c2p_tile<T, LAST>(R[m.run], ctl, m.tile, buf, false, smin, ssum);
@@ -984,7 +987,7 @@ __global__ void __launch_bounds__(256) kb_c2p(const RunArgs<T> *R, const ItemLis
 // Compaction of the runs that flagged cells this stage (one block): run list and, per class,
 // the exclusive prefix of their tiles.
 template <class T>
-__global__ void __launch_bounds__(1024) kb_fofc_scan(const RunArgs<T> *R, const int *nruns, const CondList C) {
+__global__ void __launch_bounds__(1024) kb_fofc_scan(const RunArgs<T> *__restrict__ R, const int *nruns, const CondList C) {
   constexpr int NC = CL_N + 1;   // flagged-run count + the classes
   __shared__ int s_tot[NC];
   __shared__ int s_wave[16][NC];
@@ -1063,23 +1066,23 @@ __device__ __forceinline__ void cond_walk(const CondList &C, int cls, F fn) {
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) kb_corner_cond(const RunArgs<T> *R, const CondList C) {
+__global__ void __launch_bounds__(256) kb_corner_cond(const RunArgs<T> *__restrict__ R, const CondList C) {
   cond_walk(C, CL_CORNER, [&](int r, int tile) {
     const Ctrl *ctl = R[r].ctrl;
-    const CornerArgsT<T> a = R[r].corner[ctl->wcur];
+    const CornerArgsT<T> a = R[r].corner[uniform(ctl->wcur)];
     const int t = tile * 256 + int(threadIdx.x);
     if (t < ctl->nbad * 8) corner_list_entry(a, R[r].badlist, t);
   });
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) kb_update_cond(const RunArgs<T> *R, const CondList C, int out, double g0,
+__global__ void __launch_bounds__(256) kb_update_cond(const RunArgs<T> *__restrict__ R, const CondList C, int out, double g0,
                                                       double g1, double beta) {
   cond_walk(C, CL_UPDATE, [&](int r, int tile) { update_tile(R[r], R[r].ctrl, tile, out, g0, g1, beta); });
 }
 
 template <class T, bool LAST>
-__global__ void __launch_bounds__(256) kb_c2p_cond(const RunArgs<T> *R, const CondList C, int buf) {
+__global__ void __launch_bounds__(256) kb_c2p_cond(const RunArgs<T> *__restrict__ R, const CondList C, int buf) {
   __shared__ double smin[BX * BY / 64];
   __shared__ int ssum[BX * BY / 64];
   cond_walk(C, CL_C2P, [&](int r, int tile) { c2p_tile<T, LAST>(R[r], R[r].ctrl, tile, buf, true, smin, ssum); });
@@ -1091,7 +1094,7 @@ __global__ void __launch_bounds__(256) kb_c2p_cond(const RunArgs<T> *R, const Co
 // phases; a run that flagged nothing exits at once. The tile bodies are those of the
 // multi-launch branch, so every value is the same.
 template <class T, bool LAST>
-__global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *R, const int *nruns, int out, double g0,
+__global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *__restrict__ R, const int *nruns, int out, double g0,
                                                     double g1, double beta) {
   __shared__ double smin[BX * BY / 64];
   __shared__ int ssum[BX * BY / 64];
@@ -1102,7 +1105,7 @@ __global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *R, const i
   if (!ctl->active || ctl->nbad == 0) return;   // the same for every thread of the block
   const int nbad = ctl->nbad;
   {
-    const CornerArgsT<T> a = run.corner[ctl->wcur];
+    const CornerArgsT<T> a = run.corner[uniform(ctl->wcur)];
     for (int t = int(threadIdx.x); t < nbad * 8; t += 256) corner_list_entry(a, run.badlist, t);
   }
   __syncthreads();
@@ -1113,7 +1116,7 @@ __global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *R, const i
 
 // live[r] (end of step) = 1 while run r has not reached tlim / nlim
 template <class T>
-__global__ void __launch_bounds__(256) kb_ctrl(const RunArgs<T> *R, const int *nruns, int op, int arg, int *live) {
+__global__ void __launch_bounds__(256) kb_ctrl(const RunArgs<T> *__restrict__ R, const int *nruns, int op, int arg, int *live) {
   const int r = int(blockIdx.x) * 256 + int(threadIdx.x);
   if (r >= *nruns) return;
   Ctrl *c = R[r].ctrl;
@@ -1276,19 +1279,19 @@ hipError_t launch_ctrl_turn(Ctrl *c, const CtrlTurn &t, hipStream_t s) {
 // ---------------------------------------------------------------- batched launches
 template <class T>
 hipError_t launchb_corner(const RunArgs<T> *R, ItemList L, int grid, hipStream_t s) {
-  hipLaunchKernelGGL(kb_corner<T>, dim3(grid), dim3(256), 0, s, R, L);
+  hipLaunchKernelGGL(kb_corner<T>, dim3(grid), dim3(256), 0, s, R, L.item, L.n);
   return hipGetLastError();
 }
 template <class T>
 hipError_t launchb_update(const RunArgs<T> *R, ItemList L, int out, double g0, double g1, double beta, int grid,
                           hipStream_t s) {
-  hipLaunchKernelGGL(kb_update<T>, dim3(grid), dim3(256), 0, s, R, L, out, g0, g1, beta);
+  hipLaunchKernelGGL(kb_update<T>, dim3(grid), dim3(256), 0, s, R, L.item, L.n, out, g0, g1, beta);
   return hipGetLastError();
 }
 template <class T>
 hipError_t launchb_c2p(const RunArgs<T> *R, ItemList L, int buf, int last, int grid, hipStream_t s) {
-  if (last) hipLaunchKernelGGL((kb_c2p<T, true>), dim3(grid), dim3(256), 0, s, R, L, buf);
-  else hipLaunchKernelGGL((kb_c2p<T, false>), dim3(grid), dim3(256), 0, s, R, L, buf);
+  if (last) hipLaunchKernelGGL((kb_c2p<T, true>), dim3(grid), dim3(256), 0, s, R, L.item, L.n, buf);
+  else hipLaunchKernelGGL((kb_c2p<T, false>), dim3(grid), dim3(256), 0, s, R, L.item, L.n, buf);
   return hipGetLastError();
 }
 template <class T>
