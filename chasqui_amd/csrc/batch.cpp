@@ -162,7 +162,7 @@ struct Batch final : BatchBase {
       return gx * gy * gz;
     }
     switch (k) {
-      case K_CORNER: return corner_vb(g).n;
+      case K_CORNER: return g.three_d ? corner_vb(g).n : 0;   // below 3D: part of the update
       case K_UPDATE: return update_vb(g).n;
       case K_C2P: return ghost_tiles(g) + active_vb(g).n;
       default: return 0;   // K_BC1..3: the ghost fill is part of con2prim's launch
@@ -235,8 +235,8 @@ struct Batch final : BatchBase {
     return CHQ_OK;
   }
 
-  // The launches of a stage; flux classes that no run of the batch has (the y and z
-  // directions of 1D runs, z of 2D) are left out (present[], fixed when the step is enqueued or
+  // The launches of a stage; classes that no run of the batch has (the y and z fluxes
+  // of 1D runs, z of 2D, the corner EMF launch of 3D) are left out (present[], fixed when the step is enqueued or
   // captured; a change re-captures the graph). The control launches between stages are merged:
   // begin step + begin stage 1, end stage + begin next, end last stage + end step.
   int enqueue_stage(int s) {
@@ -248,7 +248,7 @@ struct Batch final : BatchBase {
     const int *g = b->grid;
     for (int d = 0; d < 3; ++d)
       if (present[K_FLUX1 + d]) HIPCHK(launchb_flux(d_runs, list(K_FLUX1 + d), d, cf.cur, rc, rs, g[K_FLUX1 + d], st));
-    HIPCHK(launchb_corner<T>(d_runs, list(K_CORNER), g[K_CORNER], st));
+    if (present[K_CORNER]) HIPCHK(launchb_corner<T>(d_runs, list(K_CORNER), g[K_CORNER], st));
     HIPCHK(launchb_update<T>(d_runs, list(K_UPDATE), cf.out, cf.g0, cf.g1, cf.beta, g[K_UPDATE], st));
     HIPCHK(launchb_c2p<T>(d_runs, list(K_C2P), cf.out, last, g[K_C2P], st));
     // fofc branch of the runs that flagged cells: for batches of small runs, one block per run
@@ -259,7 +259,7 @@ struct Batch final : BatchBase {
     } else {
       HIPCHK(launchb_fofc_scan<T>(d_runs, d_count, cond(), st));
       HIPCHK(launchb_repair(d_runs, cond(), cf.cur, g[G_REPAIR], st));
-      HIPCHK(launchb_corner_cond<T>(d_runs, cond(), g[G_REPAIR], st));
+      if (present[K_CORNER]) HIPCHK(launchb_corner_cond<T>(d_runs, cond(), g[G_REPAIR], st));
       HIPCHK(launchb_update_cond<T>(d_runs, cond(), cf.out, cf.g0, cf.g1, cf.beta, g[G_COND], st));
       HIPCHK(launchb_c2p_cond<T>(d_runs, cond(), cf.out, last, g[G_COND], st));
     }

@@ -745,9 +745,14 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
       for (int d = 0; d < c->ndir(); ++d) HIPCHK(launch_limit_fluxes(sa, d, c->stream));
     }
   }
-  c->tmark(CHQ_K_CORNER, true);
-  HIPCHK(launch_corner<T>(c->corner_args_t(fs, wc, k, 0), c->stream));
-  c->tmark(CHQ_K_CORNER, false);
+  const CornerArgsT<T> ce = c->corner_args_t(fs, wc, k, 0);
+  const bool corn = update_has_corner(c->g, fp64);
+  const CornerArgsT<T> *uce = corn ? &ce : nullptr;   // the update launch forms the edge EMFs
+  if (!corn) {
+    c->tmark(CHQ_K_CORNER, true);
+    HIPCHK(launch_corner<T>(ce, c->stream));
+    c->tmark(CHQ_K_CORNER, false);
+  }
   const bool strict = fp64 && c->cfg.fofc && (lim || c->eos.dual_energy);
   // The first stage of RK2 and RK3 (u0 -> u1 with g1 = 0) re-updates only the points around the
   // flagged cells when it fires (k_mark_near / k_update_near), unless its first pass counted a
@@ -764,7 +769,7 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
     ua.zcount = &k->zsens;
   }
   c->tmark(CHQ_K_UPDATE, true);
-  HIPCHK(launch_update<T>(ua, c->stream));
+  HIPCHK(launch_update<T>(ua, c->stream, uce));
   c->tmark(CHQ_K_UPDATE, false);
   if (fp64 && c->gravity()) HIPCHK(launch_gravity(c->src_args(cf.out, wc, k, cf.beta, true), c->stream));   // main.cpp:76
   // Strict order (flux limiter or dual energy on): the cells are flagged here, before the
@@ -820,16 +825,16 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
       fr[d].entropy = c->entropy;
     }
     HIPCHK(launch_repair_list(fr, c->ndir(), c->badlist, c->stream));
-    HIPCHK(launch_corner_list<T>(c->corner_args_t(fs, wc, k, 1), c->badlist, c->stream));
+    if (!corn) HIPCHK(launch_corner_list<T>(c->corner_args_t(fs, wc, k, 1), c->badlist, c->stream));
     UpdateArgsT<T> ub = c->update_args_t(fs, cf.out, cf.g0, cf.g1, nvar, k, 1);
     ub.use_ctrl_dt = 1;
     ub.beta = cf.beta;
     if (local) {
       HIPCHK(launch_mark_near(c->g, k, c->badlist, c->near_marks(), c->stream));   // gate 5
-      HIPCHK(launch_update_near<T>(ub, c->near_marks(), c->stream));               // gate 5
+      HIPCHK(launch_update_near<T>(ub, uce, c->near_marks(), c->stream));               // gate 5
       ub.only_if_bad = 6;   // the whole domain when the first pass counted a point
     }
-    HIPCHK(launch_update<T>(ub, c->stream));
+    HIPCHK(launch_update<T>(ub, c->stream, uce));
     if (fp64 && c->gravity()) {   // main.cpp:89
       SrcArgs sb = c->src_args(cf.out, wc, k, cf.beta, true);
       sb.only_if_bad = 1;

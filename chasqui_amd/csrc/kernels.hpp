@@ -146,7 +146,9 @@ __host__ __device__ __forceinline__ int xcd_tile(int b, int n, int grp) {
 // con2prim 32 (1.65 -> 1.58 / 1.28 -> 1.16; 4, 8, 16 and 64 gain less), corner EMF 4 (1.47 ->
 // 1.44 / 0.90 -> 0.88; 8 and 16 the same), the float update march 8 (2.62 -> 2.60); the FP64
 // update keeps the launch order (runs of 2, 3, 4, 8 or 16 made it 0.4-1.2% slower).
-constexpr int XG_C2P = 32, XG_CORNER = 4, XG_UPDATE_F32 = 8;
+// The update that forms the edge EMFs itself (1D, 2D): 32 (512^2 mixed 11.72 -> 11.59 ms per pass,
+// 1000x1024 FP64 27.15 -> 26.96); the batched update: 8 (48 vortices FP64 135.0 -> 134.4 ms).
+constexpr int XG_C2P = 32, XG_CORNER = 4, XG_UPDATE_F32 = 8, XG_UPDATE_CORN = 32, XG_UPDATE_BATCH = 8;
 
 struct VB {
   int nx, ny, cpp, n;   // plane size, chunks per plane, total chunks
@@ -173,6 +175,14 @@ inline __host__ __device__ VB corner_vb(const Geom &g) {
 // update: active cells plus the upper faces of the present directions
 inline __host__ __device__ VB update_vb(const Geom &g) {
   return vgrid(g.ie - g.is + 2, g.two_d ? g.je - g.js + 2 : 1, g.three_d ? g.ke - g.ks + 2 : 1);
+}
+
+// Whether the update launch forms the edge EMFs: below 3D, in FP64 up to 2048 tiles. Above that the
+// 127 VGPRs of the FP64 form (96 without) cost more than the launch it saves: 1000x1024 26.96 ms
+// per pass against 26.72 with a corner launch, 700x720 10.2 against 10.8, 150x129 7.3 against 7.8;
+// mixed 512^2 11.5 against 12.0, 1024x1000 13.3 against 13.6.
+inline bool update_has_corner(const Geom &g, bool fp64) {
+  return !g.three_d && (!fp64 || update_vb(g).n <= 2048);
 }
 // con2prim: every cell, ghosts included
 inline __host__ __device__ VB c2p_vb(const Geom &g) { return vgrid(g.ni, g.nj, g.nk); }
@@ -318,14 +328,17 @@ hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int 
 hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, hipStream_t s);
 template <class T> hipError_t launch_corner(const CornerArgsT<T> &a, hipStream_t s);
 template <class T> hipError_t launch_corner_list(const CornerArgsT<T> &a, const int *list, hipStream_t s);
-template <class T> hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s);
+// with `ca` (1D and 2D meshes, update_has_corner) the launch forms the edge EMFs itself
+template <class T>
+hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s, const CornerArgsT<T> *ca = nullptr);
 // u[IENT] = rho p / rho^gamma over every cell of buffer a.u with con2prim's expressions (the
 // deferred resynchronisation of the fast path's last stage); writes nothing else
 hipError_t launch_ient_sync(const C2pArgsT<double> &a, hipStream_t s);
 // the local fofc re-update: stamp the points of the update box within one cell of each listed
 // (flagged) cell with the control block's epoch, then recompute exactly the stamped points
 hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, int *marks, hipStream_t s);
-template <class T> hipError_t launch_update_near(const UpdateArgsT<T> &a, const int *marks, hipStream_t s);
+template <class T>
+hipError_t launch_update_near(const UpdateArgsT<T> &a, const CornerArgsT<T> *ca, const int *marks, hipStream_t s);
 hipError_t launch_fill(const BcArgs &a, hipStream_t s);
 
 // explicit diffusion (FP64 single-mesh path), diffusion.hip

@@ -81,6 +81,18 @@ __device__ __forceinline__ void corner3_at(const CornerArgsT<T> &a, int k, int j
   }
 }
 
+// E3 at (j-1/2, i-1/2) of entry c, 2D (physics.hpp:288-296)
+template <class T>
+__device__ __forceinline__ T corner_e3(const CornerArgsT<T> &a, const long long c) {
+  const long long sj = a.g.pitch;
+  const T *ez = a.ecc + 2 * a.g.cstride;
+  const T l2 = upw(a.f1[c - sj], a.e3x2[c - 1] - ez[c - sj - 1], a.e3x2[c] - ez[c - sj]);
+  const T r2 = upw(a.f1[c], a.e3x2[c - 1] - ez[c - 1], a.e3x2[c] - ez[c]);
+  const T l1 = upw(a.f2[c - 1], a.e3x1[c - sj] - ez[c - sj - 1], a.e3x1[c] - ez[c - 1]);
+  const T r1 = upw(a.f2[c], a.e3x1[c - sj] - ez[c - sj], a.e3x1[c] - ez[c]);
+  return T(0.25) * (((l2 + r2) + (l1 + r1)) + ((a.e3x2[c - 1] + a.e3x2[c]) + (a.e3x1[c - sj] + a.e3x1[c])));
+}
+
 // 2D and 1D: E1/E2 are copies of the face EMFs on the two k-planes (physics.hpp:250-256);
 // E3 is the Gardiner-Stone average in 2D (288-296) or a copy in 1D (257-261).
 template <class T>
@@ -93,12 +105,7 @@ __device__ __forceinline__ void corner12_at(const CornerArgsT<T> &a, int j, int 
   a.e2[c] = a.e2x1[c];
   a.e2[c + sk] = a.e2x1[c];
   if (g.two_d) {
-    const T *ez = a.ecc + 2 * cs;
-    const T l2 = upw(a.f1[c - sj], a.e3x2[c - 1] - ez[c - sj - 1], a.e3x2[c] - ez[c - sj]);
-    const T r2 = upw(a.f1[c], a.e3x2[c - 1] - ez[c - 1], a.e3x2[c] - ez[c]);
-    const T l1 = upw(a.f2[c - 1], a.e3x1[c - sj] - ez[c - sj - 1], a.e3x1[c] - ez[c - 1]);
-    const T r1 = upw(a.f2[c], a.e3x1[c - sj] - ez[c - sj], a.e3x1[c] - ez[c]);
-    a.e3[c] = T(0.25) * (((l2 + r2) + (l1 + r1)) + ((a.e3x2[c - 1] + a.e3x2[c]) + (a.e3x1[c - sj] + a.e3x1[c])));
+    a.e3[c] = corner_e3(a, c);
   } else if (j == g.js) {
     a.e3[c] = a.e3x1[c];
     a.e3[c + sj] = a.e3x1[c];
@@ -156,9 +163,19 @@ __global__ void __launch_bounds__(256) k_corner_list(const CornerArgsT<T> a, con
 // after. With the dimensionality a template argument the loads of all variables form one
 // straight run and are in flight together (per variable, behind runtime 2D / 3D tests, each
 // round of loads waited for the one before).
-template <class T, int DIM>
-__device__ __forceinline__ void update_at_d(const UpdateArgsT<T> &a, const double bdt, int k, int j, int i) {
+// CORN (1D, 2D): the edge EMFs come from the face EMFs in the same thread instead of from a corner
+// EMF launch before. A point computes the two or three E3 it needs (the neighbours' again, from
+// cached lines) and stores its own E1, E2 and E3, the values corner12_at stores. It saves a
+// dependent launch and the round trip of five edge values per point, and a second launch in the
+// fofc branch, whose re-update then sees the repaired faces by itself. ms per pass against the
+// separate launch: 50 steps of 150x129 FP64 7.78 -> 7.29, 50 of 512^2 mixed 12.1 -> 11.6, 60 of a
+// 1D mixed run of 3999 cells 5.5 -> 4.8, 100 of 64 small mixed runs 29.7 -> 28.3 (sizes where the
+// separate launch stays: update_has_corner).
+template <class T, int DIM, bool CORN>
+__device__ __forceinline__ void update_at_d(const UpdateArgsT<T> &a, const CornerArgsT<T> &ca, const double bdt, int k,
+                                            int j, int i) {
   constexpr bool two_d = DIM >= 2, three_d = DIM == 3;
+  static_assert(!(CORN && three_d), "3D edge EMFs come from the corner launch");
   const Geom &g = a.g;
   const double g0 = a.g0, g1 = a.g1;
   const long long c = g.at(k, j, i), sj = g.pitch, sk = g.plane, cs = g.cstride;
@@ -187,21 +204,36 @@ __device__ __forceinline__ void update_at_d(const UpdateArgsT<T> &a, const doubl
   }
   double e3j = 0.0, e2k = 0.0, e3i = 0.0, e1k = 0.0, e2i = 0.0, e1j = 0.0;
   double b1a = 0.0, b1b = 0.0, b2a = 0.0, b2b = 0.0, b3a = 0.0, b3b = 0.0;
+  if constexpr (CORN) {
+    const T e1c = ca.e1x2[c], e2c = ca.e2x1[c], e3c = two_d ? corner_e3(ca, c) : ca.e3x1[c];
+    if (two_d && f1) e3j = double(corner_e3(ca, c + sj)) - double(e3c);
+    if (f2) e3i = double(two_d ? corner_e3(ca, c + 1) : ca.e3x1[c + 1]) - double(e3c);
+    if (f3) {
+      e2i = double(ca.e2x1[c + 1]) - double(e2c);
+      if (two_d) e1j = double(ca.e1x2[c + sj]) - double(e1c);
+    }
+    ca.e1[c] = e1c;
+    ca.e1[c + sk] = e1c;
+    ca.e2[c] = e2c;
+    ca.e2[c + sk] = e2c;
+    ca.e3[c] = e3c;
+    if (!two_d) ca.e3[c + sj] = e3c;
+  }
   if (f1) {
-    if (two_d) e3j = double(a.e3[c + sj]) - double(a.e3[c]);
+    if (two_d && !CORN) e3j = double(a.e3[c + sj]) - double(a.e3[c]);
     if (three_d) e2k = double(a.e2[c + sk]) - double(a.e2[c]);
     b1a = a.b1a[c];
     b1b = skip_b ? 0.0 : a.b1b[c];
   }
   if (f2) {
-    e3i = double(a.e3[c + 1]) - double(a.e3[c]);
+    if (!CORN) e3i = double(a.e3[c + 1]) - double(a.e3[c]);
     if (three_d) e1k = double(a.e1[c + sk]) - double(a.e1[c]);
     b2a = a.b2a[c];
     b2b = skip_b ? 0.0 : a.b2b[c];
   }
   if (f3) {
-    e2i = double(a.e2[c + 1]) - double(a.e2[c]);
-    if (two_d) e1j = double(a.e1[c + sj]) - double(a.e1[c]);
+    if (!CORN) e2i = double(a.e2[c + 1]) - double(a.e2[c]);
+    if (two_d && !CORN) e1j = double(a.e1[c + sj]) - double(a.e1[c]);
     b3a = a.b3a[c];
     b3b = skip_b ? 0.0 : a.b3b[c];
   }
@@ -258,11 +290,11 @@ __device__ __forceinline__ void update_at_d(const UpdateArgsT<T> &a, const doubl
   }
   if (zs) atomicAdd(a.zcount, 1);
 }
-template <class T>
-__device__ __forceinline__ void update_at(const UpdateArgsT<T> &a, const double bdt, int k, int j, int i) {
-  if (a.g.three_d) update_at_d<T, 3>(a, bdt, k, j, i);
-  else if (a.g.two_d) update_at_d<T, 2>(a, bdt, k, j, i);
-  else update_at_d<T, 1>(a, bdt, k, j, i);
+template <class T, bool CORN>
+__device__ __forceinline__ void update_at12(const UpdateArgsT<T> &a, const CornerArgsT<T> &ca, const double bdt, int k,
+                                            int j, int i) {
+  if (a.g.two_d) update_at_d<T, 2, CORN>(a, ca, bdt, k, j, i);
+  else update_at_d<T, 1, CORN>(a, ca, bdt, k, j, i);
 }
 
 // The same update with the variables in a runtime loop and the 2D / 3D terms behind runtime
@@ -362,7 +394,8 @@ __global__ void __launch_bounds__(256) k_mark_near(const Geom g, const Ctrl *ctl
 }
 
 template <class T>
-__global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, const VB v, const int *marks) {
+__global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, const CornerArgsT<T> ca, const int corn,
+                                                     const VB v, const int *marks) {
   if (!gate(a.ctrl, 5)) return;
   const Geom &g = a.g;
   const double bdt = a.use_ctrl_dt ? a.beta * a.ctrl->dt : a.beta_dt;
@@ -371,7 +404,9 @@ __global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, con
     int k, j, i;
     if (!v.at(vb, k, j, i)) continue;
     k += g.ks; j += g.js; i += g.is;
-    if (marks[g.at(k, j, i)] == epoch) update_at_loop(a, bdt, k, j, i);
+    if (marks[g.at(k, j, i)] != epoch) continue;
+    if (corn) update_at12<T, true>(a, ca, bdt, k, j, i);
+    else update_at_loop(a, bdt, k, j, i);
   }
 }
 
@@ -388,16 +423,16 @@ __global__ void __launch_bounds__(256) k_update(const UpdateArgsT<T> a, const VB
   }
 }
 // 1D and 2D meshes: the loads-first form
-template <class T>
-__global__ void __launch_bounds__(256) k_update_lf(const UpdateArgsT<T> a, const VB v) {
+template <class T, bool CORN>
+__global__ void __launch_bounds__(256) k_update_lf(const UpdateArgsT<T> a, const CornerArgsT<T> ca, const VB v) {
   if (!gate(a.ctrl, a.only_if_bad)) return;
   const Geom &g = a.g;
   const double bdt = a.use_ctrl_dt ? a.beta * a.ctrl->dt : a.beta_dt;
-  const int grp = int(gridDim.x) == v.n ? a.xg : 0;
+  const int grp = int(gridDim.x) == v.n ? (CORN ? XG_UPDATE_CORN : a.xg) : 0;
   for (int vb = blockIdx.x; vb < v.n; vb += gridDim.x) {
     int k, j, i;
     if (!v.at(xcd_tile(vb, v.n, grp), k, j, i)) continue;
-    update_at(a, bdt, g.ks + k, g.js + j, g.is + i);
+    update_at12<T, CORN>(a, ca, bdt, g.ks + k, g.js + j, g.is + i);
   }
 }
 
@@ -925,8 +960,7 @@ __global__ void __launch_bounds__(256) kb_corner(const RunArgs<T> *__restrict__ 
     const Geom &g = a.g;
     int k, j, i;
     if (!corner_vb(g).at(m.tile, k, j, i)) continue;
-    if (g.three_d) corner3_at(a, g.ks + k, g.js + j, g.is + i);
-    else corner12_at(a, g.js + j, g.is + i);
+    corner3_at(a, g.ks + k, g.js + j, g.is + i);   // (the list holds 3D runs)
   }
 }
 
@@ -939,7 +973,10 @@ __device__ __forceinline__ void update_tile(const RunArgs<T> &run, const Ctrl *c
   const double bdt = beta * ctl->dt;
   const Geom &g = a.g;
   int k, j, i;
-  if (update_vb(g).at(tile, k, j, i)) update_at(a, bdt, g.ks + k, g.js + j, g.is + i);
+  if (!update_vb(g).at(tile, k, j, i)) return;
+  const CornerArgsT<T> &ca = run.corner[uniform(ctl->wcur)];
+  if (g.three_d) update_at_d<T, 3, false>(a, ca, bdt, g.ks + k, g.js + j, g.is + i);
+  else update_at12<T, true>(a, ca, bdt, g.ks + k, g.js + j, g.is + i);
 }
 
 template <class T>
@@ -947,9 +984,8 @@ __global__ void __launch_bounds__(256) kb_update(const RunArgs<T> *__restrict__ 
                                                  const int *__restrict__ nitem, int out, double g0, double g1,
                                                  double beta) {
   const int n = *nitem;
-  const int grp = std::is_same<T, float>::value ? XG_UPDATE_F32 : 0;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
-    const Item m = uniform_item(item, xcd_tile(it, n, grp));
+    const Item m = uniform_item(item, xcd_tile(it, n, XG_UPDATE_BATCH));
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     update_tile(R[m.run], ctl, m.tile, out, g0, g1, beta);
@@ -1006,7 +1042,7 @@ __global__ void __launch_bounds__(1024) kb_fofc_scan(const RunArgs<T> *__restric
         const int nb = c->nbad;
         cnt[0] = 1;
         cnt[1 + CL_REPAIR] = div_up(nb * 2 * R[r].ndir, 256);
-        cnt[1 + CL_CORNER] = div_up(nb * 8, 256);
+        cnt[1 + CL_CORNER] = R[r].ndir == 3 ? div_up(nb * 8, 256) : 0;   // below 3D: in the update
         cnt[1 + CL_UPDATE] = R[r].cond_tiles[0];
         cnt[1 + CL_C2P] = R[r].cond_tiles[1];
       }
@@ -1106,7 +1142,7 @@ __global__ void __launch_bounds__(256) kb_fofc_runs(const RunArgs<T> *__restrict
   const int nbad = ctl->nbad;
   {
     const CornerArgsT<T> a = run.corner[uniform(ctl->wcur)];
-    for (int t = int(threadIdx.x); t < nbad * 8; t += 256) corner_list_entry(a, run.badlist, t);
+    for (int t = int(threadIdx.x); run.ndir == 3 && t < nbad * 8; t += 256) corner_list_entry(a, run.badlist, t);
   }
   __syncthreads();
   for (int tile = 0; tile < run.cond_tiles[0]; ++tile) update_tile(run, ctl, tile, out, g0, g1, beta);
@@ -1163,8 +1199,9 @@ hipError_t launch_corner_list(const CornerArgsT<T> &a, const int *list, hipStrea
   return hipGetLastError();
 }
 
+// `ca` (1D, 2D): the edge EMFs in the same launch
 template <class T>
-hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s) {
+hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s, const CornerArgsT<T> *ca) {
   const Geom &g = a.g;
   // the k march pays off for the float field set; with FP64 fluxes the plane-ordered tiles of
   // k_update stream HBM better (measured at 256^3: 3.34 vs 3.79 ms per step)
@@ -1177,7 +1214,8 @@ hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s) {
   }
   const VB v = update_vb(g);
   if (g.three_d) hipLaunchKernelGGL(k_update<T>, dim3(grid_of(v, a.only_if_bad)), dim3(256), 0, s, a, v);
-  else hipLaunchKernelGGL(k_update_lf<T>, dim3(grid_of(v, a.only_if_bad)), dim3(256), 0, s, a, v);
+  else if (ca) hipLaunchKernelGGL((k_update_lf<T, true>), dim3(grid_of(v, a.only_if_bad)), dim3(256), 0, s, a, *ca, v);
+  else hipLaunchKernelGGL((k_update_lf<T, false>), dim3(grid_of(v, a.only_if_bad)), dim3(256), 0, s, a, CornerArgsT<T>{}, v);
   return hipGetLastError();
 }
 
@@ -1185,8 +1223,8 @@ template hipError_t launch_corner<double>(const CornerArgsT<double> &, hipStream
 template hipError_t launch_corner<float>(const CornerArgsT<float> &, hipStream_t);
 template hipError_t launch_corner_list<double>(const CornerArgsT<double> &, const int *, hipStream_t);
 template hipError_t launch_corner_list<float>(const CornerArgsT<float> &, const int *, hipStream_t);
-template hipError_t launch_update<double>(const UpdateArgsT<double> &, hipStream_t);
-template hipError_t launch_update<float>(const UpdateArgsT<float> &, hipStream_t);
+template hipError_t launch_update<double>(const UpdateArgsT<double> &, hipStream_t, const CornerArgsT<double> *);
+template hipError_t launch_update<float>(const UpdateArgsT<float> &, hipStream_t, const CornerArgsT<float> *);
 
 hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, int *marks, hipStream_t s) {
   hipLaunchKernelGGL(k_mark_near, dim3(256), dim3(256), 0, s, g, ctrl, list, marks);
@@ -1194,13 +1232,14 @@ hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, in
 }
 
 template <class T>
-hipError_t launch_update_near(const UpdateArgsT<T> &a, const int *marks, hipStream_t s) {
+hipError_t launch_update_near(const UpdateArgsT<T> &a, const CornerArgsT<T> *ca, const int *marks, hipStream_t s) {
   const VB v = update_vb(a.g);   // a capped grid-stride grid: most points only read their mark
-  hipLaunchKernelGGL(k_update_near<T>, dim3(grid_of(v, true)), dim3(256), 0, s, a, v, marks);
+  hipLaunchKernelGGL(k_update_near<T>, dim3(grid_of(v, true)), dim3(256), 0, s, a, ca ? *ca : CornerArgsT<T>{},
+                     ca ? 1 : 0, v, marks);
   return hipGetLastError();
 }
-template hipError_t launch_update_near<double>(const UpdateArgsT<double> &, const int *, hipStream_t);
-template hipError_t launch_update_near<float>(const UpdateArgsT<float> &, const int *, hipStream_t);
+template hipError_t launch_update_near<double>(const UpdateArgsT<double> &, const CornerArgsT<double> *, const int *, hipStream_t);
+template hipError_t launch_update_near<float>(const UpdateArgsT<float> &, const CornerArgsT<float> *, const int *, hipStream_t);
 
 hipError_t launch_fill(const BcArgs &a, hipStream_t s) {
   hipLaunchKernelGGL(k_fill, dim3(div_up(ghost_points(a.g), 256)), dim3(256), 0, s, a);
