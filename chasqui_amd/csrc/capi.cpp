@@ -729,12 +729,22 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
   Ctrl *k = c->ctrl;
   const int nvar = c->entropy ? 6 : 5;
   const int wc = c->wcur, wn = c->wcur ^ 1;
+  FluxArgsT<T> fa[3];
   for (int d = 0; d < c->ndir(); ++d) {
-    FluxArgsT<T> fa = c->flux_args_t(fs, d, cf.cur, wc, k);
-    fa.entropy = c->entropy;
+    fa[d] = c->flux_args_t(fs, d, cf.cur, wc, k);
+    fa[d].entropy = c->entropy;
+  }
+  if (fluxk::flux_merge(fa, c->ndir(), rc, c->entropy)) {
+    fluxk::joint_seg(fa, c->ndir());
     c->tmark(CHQ_K_FLUX, true);
-    HIPCHK(launch_flux(fa, d, rc, rs, c->entropy, c->stream));
+    HIPCHK(launch_flux_all(fa, c->ndir(), rc, rs, c->entropy, c->stream));
     c->tmark(CHQ_K_FLUX, false);
+  } else {
+    for (int d = 0; d < c->ndir(); ++d) {
+      c->tmark(CHQ_K_FLUX, true);
+      HIPCHK(launch_flux(fa[d], d, rc, rs, c->entropy, c->stream));
+      c->tmark(CHQ_K_FLUX, false);
+    }
   }
   // flux limiter and gravity (FP64 contexts only) read the stage-input primitives, set wc
   constexpr bool fp64 = std::is_same<T, double>::value;
@@ -819,12 +829,7 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
   c->tmark(CHQ_K_C2P, false);
   if (c->cfg.fofc) {
     c->tmark(CHQ_K_REPAIR, true);
-    FluxArgsT<T> fr[3];
-    for (int d = 0; d < c->ndir(); ++d) {
-      fr[d] = c->flux_args_t(fs, d, cf.cur, wc, k);
-      fr[d].entropy = c->entropy;
-    }
-    HIPCHK(launch_repair_list(fr, c->ndir(), c->badlist, c->stream));
+    HIPCHK(launch_repair_list(fa, c->ndir(), c->badlist, c->stream));
     if (!corn) HIPCHK(launch_corner_list<T>(c->corner_args_t(fs, wc, k, 1), c->badlist, c->stream));
     UpdateArgsT<T> ub = c->update_args_t(fs, cf.out, cf.g0, cf.g1, nvar, k, 1);
     ub.use_ctrl_dt = 1;

@@ -36,6 +36,12 @@ hipError_t launch_flux(const FluxArgsT<double> &a, int dir, Recon rc, RSolver rs
   return fluxk::launch_flux_t<double>(a, dir, rc, rs, entropy, s);
 }
 
+hipError_t launch_flux_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s) {
+  if (a[0].charac) return launch_flux_charac_all(a, ndir, rc, rs, entropy, s);
+  if (entropy) return hipErrorInvalidValue;   // (flux_merge leaves these to launch_flux)
+  return fluxk::launch_flux_all_t<double, false>(a, ndir, rc, rs, s);
+}
+
 hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, hipStream_t s) {
   return fluxk::launch_repair_list_t<double>(a, ndir, list, s);
 }

@@ -18,6 +18,11 @@ hipError_t launch_flux(const FluxArgsT<float> &a, int dir, Recon rc, RSolver rs,
   return fluxk::go_flux_rc<float, 2, false>(a, rc, rs, s);
 }
 
+hipError_t launch_flux_all(const FluxArgsT<float> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s) {
+  if (entropy || a[0].charac) return hipErrorInvalidValue;
+  return fluxk::launch_flux_all_t<float, false>(a, ndir, rc, rs, s);
+}
+
 hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, hipStream_t s) {
   return fluxk::launch_repair_list_t<float>(a, ndir, list, s);
 }

@@ -176,10 +176,7 @@ __device__ __forceinline__ void charac_cell(const double (&r)[5][8], double bxn,
 
 // ---------------------------------------------------------------- x faces: lane = cell
 template <Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(256) k_fluxc_x(const FluxArgsT<double> a, const int nseg, const int nwaves) {
-  if (!a.ctrl->active) return;
-  const int wave = int(blockIdx.x) * 4 + int(threadIdx.x >> 6);
-  if (wave >= nwaves) return;
+__device__ __forceinline__ void fluxc_x_wave(const FluxArgsT<double> &a, const int nseg, const int wave) {
   constexpr int NV = ENT ? 8 : 7;
   constexpr bool W = wide_v<RC>;
   constexpr int H = W ? 3 : 2;
@@ -229,16 +226,21 @@ __global__ void __launch_bounds__(256) k_fluxc_x(const FluxArgsT<double> a, cons
   solve_store<double, 0, RS, ENT, NV>(a, row0 + ci, 1, Lface, Rf);
 }
 
+template <Recon RC, RSolver RS, bool ENT>
+__global__ void __launch_bounds__(256) k_fluxc_x(const FluxArgsT<double> a, const int nseg, const int nwaves) {
+  if (!a.ctrl->active) return;
+  const int wave = int(blockIdx.x) * 4 + int(threadIdx.x >> 6);
+  if (wave < nwaves) fluxc_x_wave<RC, RS, ENT>(a, nseg, wave);
+}
+
 // ---------------------------------------------------------------- y/z faces: register march
 template <int DIR, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(BX * BY) k_fluxc_m(const FluxArgsT<double> a) {
-  if (!a.ctrl->active) return;
+__device__ __forceinline__ void fluxc_m_tile(const FluxArgsT<double> &a, const int bx) {
   constexpr int NV = ENT ? 8 : 7;
   constexpr bool W = wide_v<RC>;
   const Geom &g = a.g;
   int i, t, sg;
-  if (!m_item<double, DIR>(a, (long long)blockIdx.x * (BX * BY) + int(threadIdx.y) * BX + int(threadIdx.x), i, t, sg))
-    return;
+  if (!m_item<double, DIR>(a, (long long)bx * (BX * BY) + int(threadIdx.y) * BX + int(threadIdx.x), i, t, sg)) return;
   const int lo_d = DIR == 1 ? a.jl : a.kl, hi_d = DIR == 1 ? a.ju : a.ku;
   const int F0 = lo_d + sg * a.seg;
   const int F1 = min(F0 + a.seg - 1, hi_d);
@@ -303,6 +305,27 @@ __global__ void __launch_bounds__(BX * BY) k_fluxc_m(const FluxArgsT<double> a) 
 }
 
 template <int DIR, Recon RC, RSolver RS, bool ENT>
+__global__ void __launch_bounds__(BX * BY) k_fluxc_m(const FluxArgsT<double> a) {
+  if (!a.ctrl->active) return;
+  fluxc_m_tile<DIR, RC, RS, ENT>(a, int(blockIdx.x));
+}
+
+// all directions of a small mesh in one launch (as k_flux_all)
+template <Recon RC, RSolver RS, bool ENT>
+__global__ void __launch_bounds__(256) k_fluxc_all(const FluxArgsT<double> a0, const FluxArgsT<double> a1,
+                                                   const FluxArgsT<double> a2, const int nseg, const int nwaves,
+                                                   const int nby, const int nbz) {
+  if (!a0.ctrl->active) return;
+  const int b = int(blockIdx.x);
+  if (b < nby) fluxc_m_tile<1, RC, RS, ENT>(a1, b);
+  else if (b < nby + nbz) fluxc_m_tile<2, RC, RS, ENT>(a2, b - nby);
+  else {
+    const int wave = (b - nby - nbz) * 4 + int(threadIdx.x >> 6);
+    if (wave < nwaves) fluxc_x_wave<RC, RS, ENT>(a0, nseg, wave);
+  }
+}
+
+template <int DIR, Recon RC, RSolver RS, bool ENT>
 hipError_t go_fluxc(const FluxArgsT<double> &a, hipStream_t s) {
   const int nx = a.iu - a.il + 1, ny = a.ju - a.jl + 1, nz = a.ku - a.kl + 1;
   if (nx <= 0 || ny <= 0 || nz <= 0) return hipSuccess;
@@ -327,6 +350,33 @@ hipError_t go_fluxc_rs(const FluxArgsT<double> &a, RSolver rs, hipStream_t s) {
   }
 }
 
+template <Recon RC, bool ENT>
+hipError_t go_fluxc_all_rs(const FluxArgsT<double> a[3], int ndir, RSolver rs, hipStream_t s) {
+  int nseg, nwaves, by = 0, bz = 0, q1, q2;
+  x_shape(a[0], fpw_v<RC>, nseg, nwaves);
+  if (ndir > 1) m_shape<double, 1>(a[1], by, q1, q2);
+  if (ndir > 2) m_shape<double, 2>(a[2], bz, q1, q2);
+  const dim3 grid(by + bz + div_up(nwaves, 4)), block(256);
+  const FluxArgsT<double> &a1 = a[ndir > 1 ? 1 : 0], &a2 = a[ndir > 2 ? 2 : 0];
+  switch (rs) {
+    case RSolver::hlld: hipLaunchKernelGGL((k_fluxc_all<RC, RSolver::hlld, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz); break;
+    case RSolver::lhlld: hipLaunchKernelGGL((k_fluxc_all<RC, RSolver::lhlld, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz); break;
+    default: hipLaunchKernelGGL((k_fluxc_all<RC, RSolver::hlle, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz);
+  }
+  return hipGetLastError();
+}
+
+template <bool ENT>
+hipError_t go_fluxc_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, hipStream_t s) {
+  switch (rc) {
+    case Recon::plm: return go_fluxc_all_rs<Recon::plm, ENT>(a, ndir, rs, s);
+    case Recon::ppm: return go_fluxc_all_rs<Recon::ppm, ENT>(a, ndir, rs, s);
+    case Recon::ppmx: return go_fluxc_all_rs<Recon::ppmx, ENT>(a, ndir, rs, s);
+    case Recon::wenoz: return go_fluxc_all_rs<Recon::wenoz, ENT>(a, ndir, rs, s);
+    default: return hipErrorInvalidValue;
+  }
+}
+
 template <int DIR, bool ENT>
 hipError_t go_fluxc_rc(const FluxArgsT<double> &a, Recon rc, RSolver rs, hipStream_t s) {
   switch (rc) {
@@ -340,6 +390,10 @@ hipError_t go_fluxc_rc(const FluxArgsT<double> &a, Recon rc, RSolver rs, hipStre
 
 }  // namespace
 }  // namespace fluxk
+
+hipError_t launch_flux_charac_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, bool ent, hipStream_t s) {
+  return ent ? fluxk::go_fluxc_all<true>(a, ndir, rc, rs, s) : fluxk::go_fluxc_all<false>(a, ndir, rc, rs, s);
+}
 
 hipError_t launch_flux_charac(const FluxArgsT<double> &a, int dir, Recon rc, RSolver rs, bool ent, hipStream_t s) {
   using namespace fluxk;

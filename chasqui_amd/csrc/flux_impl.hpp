@@ -362,6 +362,21 @@ __global__ void __launch_bounds__(BX * BY) k_flux_m(const FluxArgsT<T> a) {
   flux_m_tile<T, DIR, RC, RS, ENT>(a, int(blockIdx.x));
 }
 
+// All directions of a small mesh in one launch: the y and z march blocks first (the longer ones),
+// then the x blocks (flux_merge in kernels.hpp has the rule and the figures).
+template <class T, Recon RC, RSolver RS, bool ENT>
+__global__ void __launch_bounds__(256) k_flux_all(const FluxArgsT<T> a0, const FluxArgsT<T> a1, const FluxArgsT<T> a2,
+                                                  const int nseg, const int nwaves, const int nby, const int nbz) {
+  if (!a0.ctrl->active) return;
+  const int b = int(blockIdx.x);
+  if (b < nby) flux_m_tile<T, 1, RC, RS, ENT>(a1, b);
+  else if (b < nby + nbz) flux_m_tile<T, 2, RC, RS, ENT>(a2, b - nby);
+  else {
+    const int wave = (b - nby - nbz) * 4 + int(threadIdx.x >> 6);
+    if (wave < nwaves) flux_x_wave<T, RC, RS, ENT>(a0, nseg, wave);
+  }
+}
+
 // Donor-cell HLLE flux and face EMFs of one face from the stage-input primitives
 // (fofc.hpp:76-88).
 template <class T, int DIR>
@@ -452,6 +467,33 @@ hipError_t launch_flux_t(const FluxArgsT<T> &a, int dir, Recon rc, RSolver rs, b
   if (dir == 0) return ent ? go_flux_rc<T, 0, true>(a, rc, rs, s) : go_flux_rc<T, 0, false>(a, rc, rs, s);
   if (dir == 1) return ent ? go_flux_rc<T, 1, true>(a, rc, rs, s) : go_flux_rc<T, 1, false>(a, rc, rs, s);
   return ent ? go_flux_rc<T, 2, true>(a, rc, rs, s) : go_flux_rc<T, 2, false>(a, rc, rs, s);
+}
+
+template <class T, Recon RC, bool ENT>
+hipError_t go_flux_all_rs(const FluxArgsT<T> a[3], int ndir, RSolver rs, hipStream_t s) {
+  int nseg, nwaves, by = 0, bz = 0, q1, q2;
+  x_shape(a[0], fpw_v<RC>, nseg, nwaves);
+  if (ndir > 1) m_shape<T, 1>(a[1], by, q1, q2);
+  if (ndir > 2) m_shape<T, 2>(a[2], bz, q1, q2);
+  const dim3 grid(by + bz + div_up(nwaves, 4)), block(256);
+  const FluxArgsT<T> &a1 = a[ndir > 1 ? 1 : 0], &a2 = a[ndir > 2 ? 2 : 0];
+  switch (rs) {
+    case RSolver::hlld: hipLaunchKernelGGL((k_flux_all<T, RC, RSolver::hlld, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz); break;
+    case RSolver::lhlld: hipLaunchKernelGGL((k_flux_all<T, RC, RSolver::lhlld, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz); break;
+    default: hipLaunchKernelGGL((k_flux_all<T, RC, RSolver::hlle, ENT>), grid, block, 0, s, a[0], a1, a2, nseg, nwaves, by, bz);
+  }
+  return hipGetLastError();
+}
+
+template <class T, bool ENT>
+hipError_t launch_flux_all_t(const FluxArgsT<T> a[3], int ndir, Recon rc, RSolver rs, hipStream_t s) {
+  switch (rc) {
+    case Recon::dc: return go_flux_all_rs<T, Recon::dc, ENT>(a, ndir, rs, s);
+    case Recon::plm: return go_flux_all_rs<T, Recon::plm, ENT>(a, ndir, rs, s);
+    case Recon::ppm: return go_flux_all_rs<T, Recon::ppm, ENT>(a, ndir, rs, s);
+    case Recon::ppmx: return go_flux_all_rs<T, Recon::ppmx, ENT>(a, ndir, rs, s);
+    default: return go_flux_all_rs<T, Recon::wenoz, ENT>(a, ndir, rs, s);
+  }
 }
 
 template <class T>

@@ -281,6 +281,55 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
   return sg < div_up(nd, a.seg);
 }
 
+// Whether the face fluxes of all directions go in one launch (k_flux_all, k_fluxc_all). One launch
+// saves the others' dispatch and tails and lets the x blocks fill the SIMDs that a small march
+// leaves idle; but the x waves then run at the march's occupancy (two waves per SIMD in FP64
+// instead of four, three instead of eight in FP32), which costs more once each launch fills the
+// device by itself. The limits are on the march blocks at one face per thread, both sides measured
+// (ms per RK3 step, separate -> one launch):
+//   FP64   PPM    64x56x45 (1378 blocks) 0.336 -> 0.269, 160^3 (33010) 3.93 -> 3.81, 192^3 6.28 -> 6.36;
+//                 512^2 PPMX (1030) 0.300 -> 0.264, 1000x1024 (4011) 0.723 -> 0.715, 2000^2 2.58 -> 2.64
+//          PPMX   128^3 (17032) 2.50 -> 2.48, 160^3 4.47 -> 4.60
+//          WENO-Z 512^2 (1030) 0.419 -> 0.389, 750^2 0.726 -> 0.735; 96^3 (7278) 1.64 -> 1.61, 128^3 3.40 -> 3.48
+//          characteristic PPMX 80x72x64 (3083) 1.087 -> 1.009, 96^3 2.12 -> 2.18; 500^2 0.378 -> 0.382
+//   FP32   PPM    160^3 (33010) 2.45 -> 2.36, 192^3 (56748) no gain over a whole run, 256^3 8.59 -> 8.72;
+//                 1000x1024 0.440 -> 0.427, 2000^2 1.63 -> 1.65
+//          WENO-Z 256^3 (133648) 9.62 -> 9.41, 2000^2 (15648) 1.78 -> 1.76
+template <class T>
+inline bool flux_merge(const FluxArgsT<T> *a, int ndir, Recon rc, bool entropy) {
+  if (ndir < 2 || (entropy && !a[0].charac)) return false;
+  long long blocks = 0;
+  for (int d = 1; d < ndir; ++d) {
+    const MarchShape m = march_shape(a[d].il, a[d].iu, a[d].jl, a[d].ju, a[d].kl, a[d].ku, d);
+    blocks += m.rows * m.nd / 256;
+  }
+  const bool weno = rc == Recon::wenoz, d3 = ndir == 3;
+  if (sizeof(T) == 4) return weno ? (d3 || blocks <= 16000) : blocks <= (d3 ? 40000 : 8000);
+  if (a[0].charac) return d3 && blocks <= 4500;
+  if (weno) return blocks <= (d3 ? 7500 : 1500);
+  return blocks <= (d3 ? (rc == Recon::ppmx ? 18000 : 34000) : 4500);
+}
+// The march segment of a joint launch: the candidate of least (s + 1.5) (0.5 + m), m the march
+// blocks per CU. Blocks of all lengths share a CU here, so the work term has no steps at whole
+// blocks per CU as march_seg's has; fitted to sweeps over the sizes above (1.2% from the best
+// candidate on average).
+template <class T>
+inline void joint_seg(FluxArgsT<T> *a, int ndir) {
+  static constexpr int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
+  int best = 1;
+  double least = 1e300;
+  for (const int s : cand) {
+    double blocks = 0.0;
+    for (int d = 1; d < ndir; ++d) {
+      const MarchShape m = march_shape(a[d].il, a[d].iu, a[d].jl, a[d].ju, a[d].kl, a[d].ku, d);
+      blocks += double(m.rows) * ((m.nd + s - 1) / s) / 256.0;
+    }
+    const double cost = (s + 1.5) * (0.5 + blocks / 256.0);
+    if (cost < least) { least = cost; best = s; }
+  }
+  for (int d = 1; d < ndir; ++d) a[d].seg = best;
+}
+
 }  // namespace fluxk
 
 // ---------------------------------------------------------------- batches
@@ -323,6 +372,10 @@ hipError_t launch_flux(const FluxArgsT<double> &a, int dir, Recon rc, RSolver rs
 hipError_t launch_flux(const FluxArgsT<float> &a, int dir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
 // characteristic-variable reconstruction (FP64; launch_flux forwards when a.charac is set)
 hipError_t launch_flux_charac(const FluxArgsT<double> &a, int dir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
+hipError_t launch_flux_charac_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
+// every direction in one launch (flux_merge says when; the march segments are joint_seg's)
+hipError_t launch_flux_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
+hipError_t launch_flux_all(const FluxArgsT<float> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
 hipError_t launch_repair(const FluxArgs &a, int dir, bool only_if_bad, hipStream_t s);
 hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, hipStream_t s);
 hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, hipStream_t s);
