@@ -765,7 +765,7 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
   }
   const bool strict = fp64 && c->cfg.fofc && (lim || c->eos.dual_energy);
   // The first stage of RK2 and RK3 (u0 -> u1 with g1 = 0) re-updates only the points around the
-  // flagged cells when it fires (k_mark_near / k_update_near), unless its first pass counted a
+  // flagged cells when it fires (k_update_near), unless its first pass counted a
   // point where that could differ from the whole-domain re-update (FP64; the FP32 field set's
   // update does not read u1 when g1 = 0). Needs the fast fofc order and no source term after
   // the update.
@@ -798,9 +798,9 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
   // Otherwise the order adapts on the device (ctrl_begin_stage): a stage whose counterpart in
   // the previous step flagged cells flags here, before the fill (gate 3), and skips its first
   // fill and con2prim when it flags again (gate 4); any other stage flags inside con2prim
-  // (flag mode 3).
+  // (flag mode 3), and so does every stage of a small mesh (early_flag).
   const bool adaptive = c->cfg.fofc && !strict;
-  if (adaptive) {
+  if (adaptive && early_flag(c->g)) {
     C2pArgs fl = c->c2p_args(cf.out, wc, k);   // reads the conserved state and face B only
     fl.flag_mode = 2;
     fl.only_if_bad = 3;
@@ -829,17 +829,13 @@ static int enqueue_fused_stage(chq_ctx *c, const FieldSet<T> &fs, const Coef &cf
   c->tmark(CHQ_K_C2P, false);
   if (c->cfg.fofc) {
     c->tmark(CHQ_K_REPAIR, true);
-    HIPCHK(launch_repair_list(fa, c->ndir(), c->badlist, c->stream));
+    HIPCHK(launch_repair_list(fa, c->ndir(), c->badlist, local ? c->near_marks() : nullptr, c->stream));
     if (!corn) HIPCHK(launch_corner_list<T>(c->corner_args_t(fs, wc, k, 1), c->badlist, c->stream));
     UpdateArgsT<T> ub = c->update_args_t(fs, cf.out, cf.g0, cf.g1, nvar, k, 1);
     ub.use_ctrl_dt = 1;
     ub.beta = cf.beta;
-    if (local) {
-      HIPCHK(launch_mark_near(c->g, k, c->badlist, c->near_marks(), c->stream));   // gate 5
-      HIPCHK(launch_update_near<T>(ub, uce, c->near_marks(), c->stream));               // gate 5
-      ub.only_if_bad = 6;   // the whole domain when the first pass counted a point
-    }
-    HIPCHK(launch_update<T>(ub, c->stream, uce));
+    if (local) HIPCHK(launch_update_near<T>(ub, uce, c->near_marks(), c->stream));
+    else HIPCHK(launch_update<T>(ub, c->stream, uce));
     if (fp64 && c->gravity()) {   // main.cpp:89
       SrcArgs sb = c->src_args(cf.out, wc, k, cf.beta, true);
       sb.only_if_bad = 1;
@@ -884,9 +880,11 @@ static int enqueue_step(chq_ctx *c, bool first, bool more) {
   const bool fused = !(c->diffusive() && !c->cfg.sts);
   const int nvar = c->entropy ? 6 : 5;
   const bool tail = split || (!fused && c->diffusive());   // work after the last stage
+  const bool early = early_flag(c->g);
   if (first || tail) {
     CtrlTurn t{};
     t.begin_step = t.begin_stage = 1;
+    t.stage = early ? 0 : -1;
     t.reset = nst == 1;
     HIPCHK(launch_ctrl_turn(k, t, c->stream));
   }
@@ -900,8 +898,8 @@ static int enqueue_step(chq_ctx *c, bool first, bool more) {
     turn.end_step = last && !tail;
     turn.begin_step = last && !tail && more;
     turn.begin_stage = !last || turn.begin_step;
-    turn.stage = last ? 0 : s;
-    turn.reset = turn.stage == nst - 1;
+    turn.stage = !early ? -1 : last ? 0 : s;
+    turn.reset = (last ? 0 : s) == nst - 1;
     if (fused) {
       const int rc2 = c->mixed ? enqueue_fused_stage<float>(c, c->f32, cf, last, turn)
                                : enqueue_fused_stage<double>(c, c->f64, cf, last, turn);

@@ -54,7 +54,7 @@ struct Ctrl {
   unsigned long long rho_bits;   // minimum active density of the last con2prim (parabolic dt)
   long long limiter_total;       // positivity flux-limiter activations
   int early;                     // this stage flags before the boundary fill
-  int stage;                     // RK stage index of the time loop (-1: a single-kernel entry point)
+  int stage;                     // RK stage index of the time loop (-1: never flags early)
   int fired;                     // bit s: stage s of the last step flagged cells
   int epoch;                     // stages begun since the loop started (near-marks of the local re-update)
   int done;                      // blocks of a launch that ends with a control turn (CtrlTurn)

@@ -42,8 +42,8 @@ hipError_t launch_flux_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSo
   return fluxk::launch_flux_all_t<double, false>(a, ndir, rc, rs, s);
 }
 
-hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, hipStream_t s) {
-  return fluxk::launch_repair_list_t<double>(a, ndir, list, s);
+hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, int *marks, hipStream_t s) {
+  return fluxk::launch_repair_list_t<double>(a, ndir, list, marks, s);
 }
 
 hipError_t launch_repair(const FluxArgs &a, int dir, bool only_if_bad, hipStream_t s) {

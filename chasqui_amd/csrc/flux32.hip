@@ -23,8 +23,8 @@ hipError_t launch_flux_all(const FluxArgsT<float> a[3], int ndir, Recon rc, RSol
   return fluxk::launch_flux_all_t<float, false>(a, ndir, rc, rs, s);
 }
 
-hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, hipStream_t s) {
-  return fluxk::launch_repair_list_t<float>(a, ndir, list, s);
+hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, int *marks, hipStream_t s) {
+  return fluxk::launch_repair_list_t<float>(a, ndir, list, marks, s);
 }
 
 hipError_t launchb_flux(const RunArgs<float> *R, ItemList L, int dir, int cur, Recon rc, RSolver rs, int grid, hipStream_t s) {

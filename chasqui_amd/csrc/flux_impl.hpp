@@ -409,11 +409,29 @@ __device__ __forceinline__ void repair_face(const FluxArgsT<T> &a, long long c, 
 // The repair driven by the list of flagged (active) cells that con2prim builds: every face
 // touching a listed cell — its two faces in each direction — is recomputed. A face shared by
 // two listed cells is written twice with the same value.
+// `marks` (a stage with the local re-update): the points of the update box within one cell of a
+// listed cell are stamped with the stage's epoch (several cells stamp a shared point with the
+// same value), unless the first pass counted a point that calls for the whole-domain re-update.
 template <class T>
 __global__ void __launch_bounds__(256) k_repair_list(const FluxArgsT<T> a0, const FluxArgsT<T> a1,
-                                                     const FluxArgsT<T> a2, const int *list, const int ndir) {
+                                                     const FluxArgsT<T> a2, const int *list, const int ndir,
+                                                     int *marks) {
   const Ctrl *ctl = a0.ctrl;
   if (!ctl->active || ctl->nbad == 0) return;
+  if (marks && ctl->zsens == 0) {
+    const Geom &g = a0.g;
+    const int epoch = ctl->epoch, m = ctl->nbad * 27;
+    const int ku = g.three_d ? g.ke + 1 : g.ks, ju = g.two_d ? g.je + 1 : g.js;
+    for (int t = int(blockIdx.x) * 256 + int(threadIdx.x); t < m; t += int(gridDim.x) * 256) {
+      const long long r = (long long)list[t / 27] - g.ioff;   // k * plane + j * pitch + i
+      const int o = t % 27;
+      const int k = int(r / g.plane) + o / 9 - 1;
+      const int j = int((r % g.plane) / g.pitch) + (o / 3) % 3 - 1;
+      const int i = int(r % g.pitch) + o % 3 - 1;
+      if (k < g.ks || k > ku || j < g.js || j > ju || i < g.is || i > g.ie + 1) continue;
+      marks[g.at(k, j, i)] = epoch;
+    }
+  }
   const Geom &g = a0.g;
   const int per = 2 * ndir;
   const int n = ctl->nbad * per;
@@ -497,9 +515,9 @@ hipError_t launch_flux_all_t(const FluxArgsT<T> a[3], int ndir, Recon rc, RSolve
 }
 
 template <class T>
-hipError_t launch_repair_list_t(const FluxArgsT<T> a[3], int ndir, const int *list, hipStream_t s) {
+hipError_t launch_repair_list_t(const FluxArgsT<T> a[3], int ndir, const int *list, int *marks, hipStream_t s) {
   hipLaunchKernelGGL(k_repair_list<T>, dim3(256), dim3(256), 0, s, a[0], a[ndir > 1 ? 1 : 0], a[ndir > 2 ? 2 : 0],
-                     list, ndir);
+                     list, ndir, marks);
   return hipGetLastError();
 }
 

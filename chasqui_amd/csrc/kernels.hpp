@@ -377,8 +377,9 @@ hipError_t launch_flux_charac_all(const FluxArgsT<double> a[3], int ndir, Recon 
 hipError_t launch_flux_all(const FluxArgsT<double> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
 hipError_t launch_flux_all(const FluxArgsT<float> a[3], int ndir, Recon rc, RSolver rs, bool entropy, hipStream_t s);
 hipError_t launch_repair(const FluxArgs &a, int dir, bool only_if_bad, hipStream_t s);
-hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, hipStream_t s);
-hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, hipStream_t s);
+// with `marks`, also stamps the points of the local fofc re-update (k_update_near)
+hipError_t launch_repair_list(const FluxArgsT<double> a[3], int ndir, const int *list, int *marks, hipStream_t s);
+hipError_t launch_repair_list(const FluxArgsT<float> a[3], int ndir, const int *list, int *marks, hipStream_t s);
 template <class T> hipError_t launch_corner(const CornerArgsT<T> &a, hipStream_t s);
 template <class T> hipError_t launch_corner_list(const CornerArgsT<T> &a, const int *list, hipStream_t s);
 // with `ca` (1D and 2D meshes, update_has_corner) the launch forms the edge EMFs itself
@@ -387,9 +388,8 @@ hipError_t launch_update(const UpdateArgsT<T> &a, hipStream_t s, const CornerArg
 // u[IENT] = rho p / rho^gamma over every cell of buffer a.u with con2prim's expressions (the
 // deferred resynchronisation of the fast path's last stage); writes nothing else
 hipError_t launch_ient_sync(const C2pArgsT<double> &a, hipStream_t s);
-// the local fofc re-update: stamp the points of the update box within one cell of each listed
-// (flagged) cell with the control block's epoch, then recompute exactly the stamped points
-hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, int *marks, hipStream_t s);
+// the local fofc re-update: recompute the points that launch_repair_list stamped with the control
+// block's epoch (every point where the first pass counted one that needs it)
 template <class T>
 hipError_t launch_update_near(const UpdateArgsT<T> &a, const CornerArgsT<T> *ca, const int *marks, hipStream_t s);
 hipError_t launch_fill(const BcArgs &a, hipStream_t s);
@@ -453,6 +453,13 @@ hipError_t launch_ctrl_turn(Ctrl *c, const CtrlTurn &t, hipStream_t s);
 // launch ends with that control turn.
 constexpr int FILL_TURN_TILES = 2048;
 inline int fill_c2p_tiles(const Geom &g) { return ((ghost_tiles(g) + 7) & ~7) + active_vb(g).n; }
+// Whether a stage may flag early (Ctrl::early), in a launch of its own before the fill. The early
+// order saves a firing stage its second con2prim and costs every stage a launch: on meshes up to
+// EARLY_FLAG_TILES tiles the flag always stays inside con2prim. With this and the two launches that
+// the local re-update lost, ms per pass: 50 steps of 150x129 6.02 -> 5.67, 50 of 512^2 mixed 10.19 ->
+// 9.75, 40 of 64x56x45 (its first stage fires) 11.78 -> 11.43.
+constexpr int EARLY_FLAG_TILES = 2048;
+inline bool early_flag(const Geom &g) { return fill_c2p_tiles(g) > EARLY_FLAG_TILES; }
 template <class T> hipError_t launch_fill_c2p(const C2pArgsT<T> &a, hipStream_t s, const CtrlTurn *turn = nullptr);
 hipError_t launch_flag(const C2pArgs &a, hipStream_t s);   // standalone FlagBadCells
 // control-block kernels

@@ -22,16 +22,13 @@ constexpr int BX = 64, BY = 4;
 // only_if_bad: 0 always, 1 only when the stage flagged cells (the fofc branch), 2 only when it
 // flagged none (the fused stage's first boundary fill and con2prim when the flux limiter is on),
 // 3 only when the stage flags early (the flag pass before the fill), 4 unless it flagged early
-// and found cells (the first fill and con2prim of the adaptive order), 5 / 6 when it flagged
-// cells and its first pass counted no / some point the local re-update cannot skip
+// and found cells (the first fill and con2prim of the adaptive order)
 __device__ __forceinline__ bool gate(const Ctrl *c, int only_if_bad) {
   if (!c->active) return false;
   if (only_if_bad == 1 && c->nbad == 0) return false;
   if (only_if_bad == 2 && c->nbad != 0) return false;
   if (only_if_bad == 3 && !c->early) return false;
   if (only_if_bad == 4 && c->early && c->nbad != 0) return false;
-  if (only_if_bad == 5 && (c->nbad == 0 || c->zsens != 0)) return false;
-  if (only_if_bad == 6 && (c->nbad == 0 || c->zsens == 0)) return false;
   return true;
 }
 
@@ -372,39 +369,27 @@ __device__ __forceinline__ void update_at_loop(const UpdateArgsT<T> &a, const do
 // the first pass's watch counted a point (then the whole domain is recomputed instead). The
 // repair changes the fluxes of the flagged cells' faces and the EMFs of their edges, and only
 // the points of the update box within one cell of a flagged cell read those, so:
-//   k_mark_near   - stamps those points (3x3x3 around each listed cell) with the stage's epoch;
-//                   several cells stamp a shared point with the same value
+//   k_repair_list - stamps those points (3x3x3 around each listed cell) with the stage's epoch
 //   k_update_near - one thread per point of the update box recomputes the stamped ones, each
-//                   once, reading the first-pass value of the aliased buffer, as the reference
-// Stamps of earlier stages hold smaller epochs and are ignored.
-__global__ void __launch_bounds__(256) k_mark_near(const Geom g, const Ctrl *ctl, const int *list, int *marks) {
-  if (!gate(ctl, 5)) return;
-  const int epoch = ctl->epoch;
-  const int n = ctl->nbad * 27;
-  const int ku = g.three_d ? g.ke + 1 : g.ks, ju = g.two_d ? g.je + 1 : g.js;
-  for (int t = int(blockIdx.x) * 256 + int(threadIdx.x); t < n; t += int(gridDim.x) * 256) {
-    const long long r = (long long)list[t / 27] - g.ioff;   // k * plane + j * pitch + i
-    const int o = t % 27;
-    const int k = int(r / g.plane) + o / 9 - 1;
-    const int j = int((r % g.plane) / g.pitch) + (o / 3) % 3 - 1;
-    const int i = int(r % g.pitch) + o % 3 - 1;
-    if (k < g.ks || k > ku || j < g.js || j > ju || i < g.is || i > g.ie + 1) continue;
-    marks[g.at(k, j, i)] = epoch;
-  }
-}
-
+//                   once, reading the first-pass value of the aliased buffer, as the reference;
+//                   all of them where the watch counted a point (the recomputation is pointwise,
+//                   so the whole domain needs no other form)
+// Stamps of earlier stages hold smaller epochs and are ignored. With the stamps in the repair's
+// launch and both re-updates in one, a stage of this kind has two launches fewer (about 4 us each
+// on the device even when nothing was flagged).
 template <class T>
 __global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, const CornerArgsT<T> ca, const int corn,
                                                      const VB v, const int *marks) {
-  if (!gate(a.ctrl, 5)) return;
+  if (!gate(a.ctrl, 1)) return;
   const Geom &g = a.g;
   const double bdt = a.use_ctrl_dt ? a.beta * a.ctrl->dt : a.beta_dt;
   const int epoch = a.ctrl->epoch;
+  const bool whole = a.ctrl->zsens != 0;
   for (int vb = blockIdx.x; vb < v.n; vb += gridDim.x) {
     int k, j, i;
     if (!v.at(vb, k, j, i)) continue;
     k += g.ks; j += g.js; i += g.is;
-    if (marks[g.at(k, j, i)] != epoch) continue;
+    if (!whole && marks[g.at(k, j, i)] != epoch) continue;
     if (corn) update_at12<T, true>(a, ca, bdt, k, j, i);
     else update_at_loop(a, bdt, k, j, i);
   }
@@ -804,8 +789,8 @@ __device__ __forceinline__ void ctrl_begin_step(Ctrl *c) {
 // fires again it fills and converts once; other stages keep the flag inside con2prim and pay a
 // second fill and con2prim only when they fire. Firing clusters by stage (the first stage's
 // full forward step, mostly), not from one stage to the next. Both orders give the same bits:
-// boundaries never change the active cells the flag reads. stage -1 (the single-kernel entry
-// points) never flags early.
+// boundaries never change the active cells the flag reads. stage -1 (small meshes, early_flag;
+// the single-kernel entry points) never flags early.
 __device__ __forceinline__ void ctrl_begin_stage(Ctrl *c, int reset_slots, int stage) {
   c->epoch += 1;
   c->zsens = 0;
@@ -1225,11 +1210,6 @@ template hipError_t launch_corner_list<double>(const CornerArgsT<double> &, cons
 template hipError_t launch_corner_list<float>(const CornerArgsT<float> &, const int *, hipStream_t);
 template hipError_t launch_update<double>(const UpdateArgsT<double> &, hipStream_t, const CornerArgsT<double> *);
 template hipError_t launch_update<float>(const UpdateArgsT<float> &, hipStream_t, const CornerArgsT<float> *);
-
-hipError_t launch_mark_near(const Geom &g, const Ctrl *ctrl, const int *list, int *marks, hipStream_t s) {
-  hipLaunchKernelGGL(k_mark_near, dim3(256), dim3(256), 0, s, g, ctrl, list, marks);
-  return hipGetLastError();
-}
 
 template <class T>
 hipError_t launch_update_near(const UpdateArgsT<T> &a, const CornerArgsT<T> *ca, const int *marks, hipStream_t s) {
