@@ -168,6 +168,15 @@ __device__ __forceinline__ void recon_lanes(const T q[NV], const bool flatten, c
       Rf[n] = lo;
       Lf[n] = hi;
     }
+  } else if constexpr (RC == Recon::ppmx) {
+#pragma unroll
+    for (int n = 0; n < NV; ++n) {   // the edge below this cell is the lower lane's e_{c+1/2}
+      const T qm1 = lane_up(q[n]), qp1 = lane_dn(q[n]), qm2 = lane_up<2>(q[n]), qp2 = lane_dn<2>(q[n]);
+      T hi = R::xedge(qm1, q[n], qp1, qp2), lo = lane_up(hi);
+      R::xmono(qm2, qm1, q[n], qp1, qp2, lo, hi);
+      Rf[n] = lo;
+      Lf[n] = hi;
+    }
   } else {
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
@@ -260,8 +269,9 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
   const bool flat = W && a.flatten;
   const T dfl = T(a.eos.dfloor), pfl = T(a.eos.pfloor);
   // window around the cell being finished, c: x1 = q_{c-2}, x2 = q_{c-1}, w0 = q_c, wp1 = q_{c+1}
-  // (PPM keeps x1 = d_c and x2 = e_{c-1/2} instead, plus p_{c-2}, p_{c-1}, u_{c-1})
-  T w0[NV], wp1[NV], x1[NV], x2[NV];
+  // (PPM keeps x1 = d_c and x2 = e_{c-1/2} instead, plus p_{c-2}, p_{c-1}, u_{c-1}; PPMX keeps its
+  // edge e_{c-1/2} besides)
+  T w0[NV], wp1[NV], x1[NV], x2[NV], ep[NV];
   T pm2 = T(0), pm1 = T(0), um1 = T(0);
   int c = F0 - 1;
   {
@@ -286,7 +296,11 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
       um1 = qm1[1];
     } else {
 #pragma unroll
-      for (int n = 0; n < NV; ++n) { x1[n] = qm2[n]; x2[n] = qm1[n]; }
+      for (int n = 0; n < NV; ++n) {
+        x1[n] = qm2[n];
+        x2[n] = qm1[n];
+        if constexpr (RC == Recon::ppmx) ep[n] = R::xedge(qm2[n], qm1[n], w0[n], wp1[n]);
+      }
     }
   }
   T Lprev[NV];
@@ -333,7 +347,18 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
       for (int n = 0; n < NV; ++n) { x1[n] = dn[n]; x2[n] = en[n]; }
     } else {
 #pragma unroll
-      for (int n = 0; n < NV; ++n) cell_halves<T, RC>(x1[n], x2[n], w0[n], wp1[n], qn[n], Rf[n], Lf[n]);
+      for (int n = 0; n < NV; ++n) {
+        if constexpr (RC == Recon::ppmx) {
+          const T en = R::xedge(x2[n], w0[n], wp1[n], qn[n]);   // e_{c+1/2}
+          T lo = ep[n], hi = en;
+          R::xmono(x1[n], x2[n], w0[n], wp1[n], qn[n], lo, hi);
+          Rf[n] = lo;
+          Lf[n] = hi;
+          ep[n] = en;
+        } else {
+          cell_halves<T, RC>(x1[n], x2[n], w0[n], wp1[n], qn[n], Rf[n], Lf[n]);
+        }
+      }
       if (flat) fco = R::flat(x1[4], x2[4], w0[4], wp1[4], qn[4], x2[1], wp1[1]);
 #pragma unroll
       for (int n = 0; n < NV; ++n) { x1[n] = x2[n]; x2[n] = w0[n]; }

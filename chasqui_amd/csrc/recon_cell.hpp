@@ -70,8 +70,7 @@ __device__ __forceinline__ void cell_halves(T qm2, T qm1, T q0, T qp1, T qp2, T 
     Rf = lo;
     Lf = hi;
   } else {
-    Lf = R::wz(qm2, qm1, q0, qp1, qp2);
-    Rf = R::wz(qp2, qp1, q0, qm1, qm2);
+    R::wz_pair(qm2, qm1, q0, qp1, qp2, Rf, Lf);
   }
 }
 
