@@ -156,17 +156,36 @@ __device__ __forceinline__ void recon_lanes(const T q[NV], const bool flatten, c
       const T qm = lane_up(q[n]), qp = lane_dn(q[n]);
       d[n] = R::mc(qm, q[n], qp);
     }
+    T dp[NV];
+    bool oke = true, okm = true;
 #pragma unroll
     for (int n = 0; n < NV; ++n) {   // e[n] = edge at c+1/2
-      const T qp = lane_dn(q[n]), dp = lane_dn(d[n]);
-      e[n] = R::edge(q[n], qp, d[n], dp);
+      const T qp = lane_dn(q[n]);
+      dp[n] = lane_dn(d[n]);
+      e[n] = R::edge(q[n], qp, d[n], dp[n], oke);
+    }
+    if constexpr (sizeof(T) == 8) {
+      if (__builtin_amdgcn_ballot_w64(!oke)) {   // (whole waves: the lane shifts need every lane)
+#pragma unroll
+        for (int n = 0; n < NV; ++n) e[n] = R::template edge<true>(q[n], lane_dn(q[n]), d[n], dp[n], oke);
+      }
     }
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
       T lo = lane_up(e[n]), hi = e[n];
-      R::mono(q[n], lo, hi);
+      R::mono(q[n], lo, hi, okm);
       Rf[n] = lo;
       Lf[n] = hi;
+    }
+    if constexpr (sizeof(T) == 8) {
+      if (__builtin_amdgcn_ballot_w64(!okm)) {
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+          Rf[n] = lane_up(e[n]);
+          Lf[n] = e[n];
+          R::template mono<true>(q[n], Rf[n], Lf[n], okm);
+        }
+      }
     }
   } else if constexpr (RC == Recon::ppmx) {
 #pragma unroll
@@ -288,8 +307,9 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         const T dm = R::mc(qm2[n], qm1[n], w0[n]);
+        bool ok = true;
         x1[n] = R::mc(qm1[n], w0[n], wp1[n]);            // d_c
-        x2[n] = R::edge(qm1[n], w0[n], dm, x1[n]);       // e_{c-1/2}
+        x2[n] = R::template edge<true>(qm1[n], w0[n], dm, x1[n], ok);   // e_{c-1/2}
       }
       pm2 = qm2[4];
       pm1 = qm1[4];
@@ -330,14 +350,24 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
     T Lf[NV], Rf[NV], fco = T(0);
     if constexpr (RC == Recon::ppm) {
       T dn[NV], en[NV];
+      bool ok = true;
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        dn[n] = R::mc(w0[n], wp1[n], qn[n]);             // d_{c+1}
-        en[n] = R::edge(w0[n], wp1[n], x1[n], dn[n]);    // e_{c+1/2}
+        dn[n] = R::mc(w0[n], wp1[n], qn[n]);                 // d_{c+1}
+        en[n] = R::edge(w0[n], wp1[n], x1[n], dn[n], ok);    // e_{c+1/2}
         T lo = x2[n], hi = en[n];
-        R::mono(w0[n], lo, hi);
+        R::mono(w0[n], lo, hi, ok);
         Rf[n] = lo;
         Lf[n] = hi;
+      }
+      if (!ok) {
+#pragma unroll
+        for (int n = 0; n < NV; ++n) {
+          en[n] = R::template edge<true>(w0[n], wp1[n], x1[n], dn[n], ok);
+          Rf[n] = x2[n];
+          Lf[n] = en[n];
+          R::template mono<true>(w0[n], Rf[n], Lf[n], ok);
+        }
       }
       if (flat) fco = R::flat(pm2, pm1, w0[4], wp1[4], qn[4], um1, wp1[1]);
       pm2 = pm1;

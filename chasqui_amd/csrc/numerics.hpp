@@ -37,21 +37,57 @@ CHQ_FN float vmax(float a, float b) { return fmaxf(a, b); }
 CHQ_FN float vabs(float a) { return fabsf(a); }
 CHQ_FN float vsqrt(float a) { return sqrtf(a); }
 
+// Computes v here: without it the compiler moves a variable's arithmetic down to where its result
+// is used, past the next variables', and every variable's intermediate values are live at once.
+CHQ_FN void pin(double &v) {
+#ifdef __HIP_DEVICE_COMPILE__
+  asm volatile("" : "+v"(v));
+#else
+  (void)v;
+#endif
+}
+CHQ_FN void pin(float &) {}
+
+// v (not negative) with the sign of s
+CHQ_FN double vcopysign(double v, double s) { return copysign(v, s); }
+CHQ_FN float vcopysign(float v, float s) { return sgn(s) * v; }   // (s != 0 where it is used)
+
 // x / 6, rounded exactly as the division is (the reconstructions divide by 6 up to eight times
 // per variable and cell). Markstein's theorem: with y = RN(1/6) (relative error < 2^-53) the
-// product q = RN(x * y) is within one ulp of x/6, the remainder r = x - 6q is exact in one FMA,
-// and RN(q + r * y) is the correctly rounded quotient, provided nothing underflows or
-// overflows: three instructions in place of the ~11 of a general FP64 division. Zeros return
-// q (which keeps the sign); tiny, huge and non-finite x take the division.
-CHQ_FN double div6(double x) {
+// product q = RN(x * y) is within one ulp of x/6, the remainder 6q - x is exact in one FMA (a
+// multiple of q's last place, a few of them at most), and q less y times the remainder, rounded
+// once, is the correctly rounded quotient while q is normal: three instructions in place of the ~11
+// of a general FP64 division. With the remainder in this sign a zero x keeps its sign (q is the
+// result: the remainder is +0), and an x that underflows to q = 0 is within half of the smallest
+// denormal of 0 after the division too. A denormal q (where a quotient can be a tie) or one that
+// is not finite needs the division: div6_fast reports it by clearing `ok`, so a run of quotients
+// is tested once and formed again by division where that is needed, and the common path has no
+// branch between them.
+CHQ_FN double div6_fast(double x, bool &ok) {
   constexpr double y = 1.0 / 6.0;
-  const double ax = fabs(x);
   const double q = x * y;
-  if (ax >= 0x1p-900 && ax <= 0x1p1000) return fma(fma(-6.0, q, x), y, q);
-  if (ax == 0.0) return q;
-  return x / 6.0;
+#ifdef __HIP_DEVICE_COMPILE__
+  ok = ok & __builtin_amdgcn_class(q, 0x168);   // normal or zero, of either sign
+#else
+  ok = ok && (q == 0.0 || std::isnormal(q));
+#endif
+  return fma(-y, fma(6.0, q, -x), q);
 }
-CHQ_FN float div6(float x) { return x / 6.0f; }
+CHQ_FN float div6_fast(float x, bool &) { return x / 6.0f; }
+// the division itself, in div6_fast's form
+CHQ_FN double div6_full(double x, bool &) { return x / 6.0; }
+CHQ_FN float div6_full(float x, bool &) { return x / 6.0f; }
+template <class T>
+CHQ_FN T div6(T x) {
+  bool ok = true;
+  const T r = div6_fast(x, ok);
+  return ok ? r : div6_full(x, ok);
+}
+template <bool FULL, class T>
+CHQ_FN T div6_as(T x, bool &ok) {
+  if constexpr (FULL) return div6_full(x, ok);
+  else return div6_fast(x, ok);
+}
 
 // ----------------------------------------------------------------- reconstruction
 // s[0..5] = cells i-3..i+2 around face i-1/2; L = right value of cell i-1, R = left
@@ -65,19 +101,46 @@ template <class T> struct Rec {
   // MC slope, recon.hpp:21-27
   static CHQ_FN T mc(T a, T b, T c) {
     const T l = b - a, r = c - b;
-    if (l * r <= T(0)) return T(0);
+    if constexpr (sizeof(T) == 4) {
+      if (l * r <= T(0)) return T(0);
+      const T m = T(0.5) * (c - a);
+      const T cap = T(2) * vmin(vabs(l), vabs(r));
+      return sgn(m) * vmin(vabs(m), cap);
+    }
+    // where the product is positive m is not zero, so copysign is the reference's sgn(m) * (...)
     const T m = T(0.5) * (c - a);
     const T cap = T(2) * vmin(vabs(l), vabs(r));
-    return sgn(m) * vmin(vabs(m), cap);
+    return l * r > T(0) ? vcopysign(vmin(vabs(m), cap), m) : T(0);
   }
+  // The FP64 CW84 steps hold one branch per cell and variable (the extremum test, which lets the
+  // waves of a uniform region leave early) instead of six: a divergent branch costs the wave its
+  // exec-mask updates and a jump, and it keeps the seven variables' independent chains from
+  // overlapping. Face fluxes at 256^3 (blast, mostly uniform): x 718 -> 681 us, y 782 -> 733, z 731 ->
+  // 688; 128^3 wave, all directions 393 -> 365. Without the extremum's branch the wave is as fast and
+  // the blast slower (727, 784, 737). FP32 keeps the branches (FMA contraction would follow the new
+  // form's other uses of the products, and the results would be other ones). FULL: by division (div6_fast's
+  // fallback).
   // CW84 interface, recon.hpp:42-44
-  static CHQ_FN T edge(T qa, T qb, T da, T db) { return T(0.5) * (qa + qb) + div6(da - db); }
+  template <bool FULL = false>
+  static CHQ_FN T edge(T qa, T qb, T da, T db, bool &ok) {
+    return T(0.5) * (qa + qb) + div6_as<FULL>(da - db, ok);
+  }
   // CW84 monotonization, recon.hpp:47-57
-  static CHQ_FN void mono(T q, T &lo, T &hi) {
+  template <bool FULL = false>
+  static CHQ_FN void mono(T q, T &lo, T &hi, bool &ok) {
+    if constexpr (sizeof(T) == 4) {
+      if ((hi - q) * (q - lo) <= T(0)) { lo = q; hi = q; return; }
+      const T d = hi - lo, c = q - T(0.5) * (lo + hi), t = div6(d * d);
+      if (d * c > t) lo = T(3) * q - T(2) * hi;
+      else if (d * c < -t) hi = T(3) * q - T(2) * lo;
+      return;
+    }
     if ((hi - q) * (q - lo) <= T(0)) { lo = q; hi = q; return; }
-    const T d = hi - lo, c = q - T(0.5) * (lo + hi), t = div6(d * d);
-    if (d * c > t) lo = T(3) * q - T(2) * hi;
-    else if (d * c < -t) hi = T(3) * q - T(2) * lo;
+    const T d = hi - lo, c = q - T(0.5) * (lo + hi), t = div6_as<FULL>(d * d, ok);
+    const bool over = d * c > t, under = !over && d * c < -t;
+    const T l = over ? T(3) * q - T(2) * hi : lo, h = under ? T(3) * q - T(2) * lo : hi;
+    lo = l;
+    hi = h;
   }
   // PPMX interface, recon.hpp:85-100
   static CHQ_FN T xedge(T qm1, T q0, T qp1, T qp2) {
@@ -88,7 +151,7 @@ template <class T> struct Rec {
       const T dl = (qm1 + qp1) - T(2) * q0;
       const T dr = (q0 + qp2) - T(2) * qp1;
       T lim = T(0);
-      if (d2 * dl > T(0) && d2 * dr > T(0)) lim = sgn(d2) * vmin(vmin(C * vabs(dl), C * vabs(dr)), vabs(d2));
+      if (d2 * dl > T(0) && d2 * dr > T(0)) lim = vcopysign(vmin(vmin(C * vabs(dl), C * vabs(dr)), vabs(d2)), d2);
       f = T(0.5) * (q0 + qp1) - div6(lim);
     }
     return f;
@@ -104,7 +167,7 @@ template <class T> struct Rec {
       const T dr = (q + qp2) - T(2) * qp1;
       T lim = T(0);
       if (d2 * dc > T(0) && d2 * dl > T(0) && d2 * dr > T(0))
-        lim = sgn(d2) * vmin(vmin(C * vabs(dl), C * vabs(dr)), vmin(C * vabs(dc), vabs(d2)));
+        lim = vcopysign(vmin(vmin(C * vabs(dl), C * vabs(dr)), vmin(C * vabs(dc), vabs(d2))), d2);
       const T rho = (vabs(d2) > Lit<T>::rel * (vabs(q) + vabs(qm1) + vabs(qp1)) + Lit<T>::tiny) ? lim / d2 : T(0);
       if (rho < T(1) - Lit<T>::rel) { lo = q - rho * dm; hi = q + rho * dp; }
     } else {
@@ -144,22 +207,27 @@ template <class T> struct Rec {
     const T tau = vabs(s0 - s2);
     const T t0 = T(1) + tau / (s0 + eps), t1 = T(1) + tau / (s1 + eps), t2 = T(1) + tau / (s2 + eps);
     const T w1 = T(0.6) * t1;
+    const T x0 = T(2) * a - T(7) * b + T(11) * c, x1 = -b + T(5) * c + T(2) * d, x2 = T(2) * c + T(5) * d - e;
+    const T z0 = T(2) * e - T(7) * d + T(11) * c, z1 = -d + T(5) * c + T(2) * b, z2 = T(2) * c + T(5) * b - a;
+    bool ok = true;
+    T p0 = div6_fast(x0, ok), p1 = div6_fast(x1, ok), p2 = div6_fast(x2, ok);
+    T r0 = div6_fast(z0, ok), r1 = div6_fast(z1, ok), r2 = div6_fast(z2, ok);
+    if (!ok) {
+      p0 = div6_full(x0, ok); p1 = div6_full(x1, ok); p2 = div6_full(x2, ok);
+      r0 = div6_full(z0, ok); r1 = div6_full(z1, ok); r2 = div6_full(z2, ok);
+    }
     {
       const T w0 = T(0.1) * t0, w2 = T(0.3) * t2;
       const T inv = T(1) / (w0 + w1 + w2);
-      const T p0 = div6(T(2) * a - T(7) * b + T(11) * c);
-      const T p1 = div6(-b + T(5) * c + T(2) * d);
-      const T p2 = div6(T(2) * c + T(5) * d - e);
       hi = inv * (w0 * p0 + w1 * p1 + w2 * p2);
     }
     {
       const T w0 = T(0.1) * t2, w2 = T(0.3) * t0;
       const T inv = T(1) / (w0 + w1 + w2);
-      const T p0 = div6(T(2) * e - T(7) * d + T(11) * c);
-      const T p1 = div6(-d + T(5) * c + T(2) * b);
-      const T p2 = div6(T(2) * c + T(5) * b - a);
-      lo = inv * (w0 * p0 + w1 * p1 + w2 * p2);
+      lo = inv * (w0 * r0 + w1 * r1 + w2 * r2);
     }
+    pin(hi);
+    pin(lo);
   }
 
   template <Recon R>
@@ -171,11 +239,12 @@ template <class T> struct Rec {
     } else if constexpr (R == Recon::ppm) {               // recon.hpp:60-78
       const T m1 = mc(s[0], s[1], s[2]), m2 = mc(s[1], s[2], s[3]);
       const T m3 = mc(s[2], s[3], s[4]), m4 = mc(s[3], s[4], s[5]);
-      const T e1 = edge(s[2], s[3], m2, m3);
-      T a = edge(s[1], s[2], m1, m2), b = e1;
-      mono(s[2], a, b);
-      T c = e1, d = edge(s[3], s[4], m3, m4);
-      mono(s[3], c, d);
+      bool ok = true;
+      const T e1 = edge<true>(s[2], s[3], m2, m3, ok);
+      T a = edge<true>(s[1], s[2], m1, m2, ok), b = e1;
+      mono<true>(s[2], a, b, ok);
+      T c = e1, d = edge<true>(s[3], s[4], m3, m4, ok);
+      mono<true>(s[3], c, d, ok);
       L = b; R_ = c;
     } else if constexpr (R == Recon::ppmx) {              // recon.hpp:129-140
       const T e1 = xedge(s[1], s[2], s[3], s[4]);

@@ -60,8 +60,14 @@ __device__ __forceinline__ void cell_halves(T qm2, T qm1, T q0, T qp1, T qp2, T 
     Rf = q0 - T(0.5) * s;
   } else if constexpr (RC == Recon::ppm) {
     const T dm = R::mc(qm2, qm1, q0), d0 = R::mc(qm1, q0, qp1), dp = R::mc(q0, qp1, qp2);
-    T lo = R::edge(qm1, q0, dm, d0), hi = R::edge(q0, qp1, d0, dp);
-    R::mono(q0, lo, hi);
+    bool ok = true;
+    T lo = R::edge(qm1, q0, dm, d0, ok), hi = R::edge(q0, qp1, d0, dp, ok);
+    R::mono(q0, lo, hi, ok);
+    if (!ok) {
+      lo = R::template edge<true>(qm1, q0, dm, d0, ok);
+      hi = R::template edge<true>(q0, qp1, d0, dp, ok);
+      R::template mono<true>(q0, lo, hi, ok);
+    }
     Rf = lo;
     Lf = hi;
   } else if constexpr (RC == Recon::ppmx) {
