@@ -266,9 +266,23 @@ __global__ void __launch_bounds__(256) k_flux_x(const FluxArgsT<T> a, const int 
 }
 
 // ---------------------------------------------------------------- y/z faces: register march
+// PARK (FP32, wide stencils): what the next cell needs besides its cells' values waits in LDS while
+// the face is solved, NPARK arrays of a thread's own entries, 28 KB a block at most. The solver is
+// where the registers peak (136 to 141, three waves per SIMD); so they fit 128, four waves. ms per
+// pass: 30 steps of 192^3 PPM 144.7 -> 142.1, 20 of 128^3 WENO-Z 34.0 -> 33.6; 2D PPMX the same. In FP64
+// the same park leaves PPM and PPMX 12 to 100 bytes over three waves' 168 registers, and the spills
+// cost more than the third wave gives (256^3: 333 -> 343 ms); at two waves it only adds LDS traffic
+// (333 -> 336).
+template <class T, Recon RC> constexpr bool park_v = sizeof(T) == 4 && wide_v<RC>;
+template <Recon RC> constexpr int npark_v = RC == Recon::ppmx ? 4 : 3;
+template <class T, Recon RC, bool ENT>
+constexpr int park_n = park_v<T, RC> ? npark_v<RC> * (ENT ? 8 : 7) * BX * BY : 1;
+template <class T, Recon RC> constexpr int march_waves_v = park_v<T, RC> ? 4 : 1;
+
 template <class T, int DIR, Recon RC, RSolver RS, bool ENT>
-__device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx) {
-  constexpr int NV = ENT ? 8 : 7;
+__device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx, T *park) {
+  constexpr int NV = ENT ? 8 : 7, SP = BX * BY;   // SP: distance of a thread's parked entries
+  constexpr bool PARK = park_v<T, RC>;
   constexpr bool W = wide_v<RC>;
   const Geom &g = a.g;
   // i, transverse index t (k for DIR 1, j for DIR 2) and segment along DIR
@@ -397,7 +411,28 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
 #pragma unroll
     for (int n = 0; n < NV; ++n) qc[n] = w0[n];
     finish_cell<T, NV>(Lf, Rf, qc, fco, flat, dfl, pfl);
+    T *const pk = park + int(threadIdx.y) * BX + int(threadIdx.x);
+    if constexpr (PARK) {
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        pk[n * SP] = Lf[n];
+        pk[(NV + n) * SP] = x1[n];
+        pk[(2 * NV + n) * SP] = x2[n];
+        if constexpr (RC == Recon::ppmx) pk[(3 * NV + n) * SP] = ep[n];
+      }
+      asm volatile("" ::: "memory");   // (nothing is forwarded past the solver in registers)
+    }
     if (c >= F0) solve_store<T, DIR, RS, ENT, NV>(a, cc, sd, Lprev, Rf);   // face c (between c-1 and c)
+    if constexpr (PARK) {
+      asm volatile("" ::: "memory");
+#pragma unroll
+      for (int n = 0; n < NV; ++n) {
+        Lf[n] = pk[n * SP];
+        x1[n] = pk[(NV + n) * SP];
+        x2[n] = pk[(2 * NV + n) * SP];
+        if constexpr (RC == Recon::ppmx) ep[n] = pk[(3 * NV + n) * SP];
+      }
+    }
     // advance the window
     if constexpr (W) {
 #pragma unroll
@@ -412,20 +447,22 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx)
 }
 
 template <class T, int DIR, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(BX * BY) k_flux_m(const FluxArgsT<T> a) {
+__global__ void __launch_bounds__(BX * BY, (march_waves_v<T, RC>)) k_flux_m(const FluxArgsT<T> a) {
+  __shared__ T park[park_n<T, RC, ENT>];
   if (!a.ctrl->active) return;
-  flux_m_tile<T, DIR, RC, RS, ENT>(a, int(blockIdx.x));
+  flux_m_tile<T, DIR, RC, RS, ENT>(a, int(blockIdx.x), park);
 }
 
 // All directions of a small mesh in one launch: the y and z march blocks first (the longer ones),
 // then the x blocks (flux_merge in kernels.hpp has the rule and the figures).
 template <class T, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(256) k_flux_all(const FluxArgsT<T> a0, const FluxArgsT<T> a1, const FluxArgsT<T> a2,
+__global__ void __launch_bounds__(256, (march_waves_v<T, RC>)) k_flux_all(const FluxArgsT<T> a0, const FluxArgsT<T> a1, const FluxArgsT<T> a2,
                                                   const int nseg, const int nwaves, const int nby, const int nbz) {
+  __shared__ T park[park_n<T, RC, ENT>];
   if (!a0.ctrl->active) return;
   const int b = int(blockIdx.x);
-  if (b < nby) flux_m_tile<T, 1, RC, RS, ENT>(a1, b);
-  else if (b < nby + nbz) flux_m_tile<T, 2, RC, RS, ENT>(a2, b - nby);
+  if (b < nby) flux_m_tile<T, 1, RC, RS, ENT>(a1, b, park);
+  else if (b < nby + nbz) flux_m_tile<T, 2, RC, RS, ENT>(a2, b - nby, park);
   else {
     const int wave = (b - nby - nbz) * 4 + int(threadIdx.x >> 6);
     if (wave < nwaves) flux_x_wave<T, RC, RS, ENT>(a0, nseg, wave);
@@ -597,15 +634,16 @@ __global__ void __launch_bounds__(256) kb_flux_x(const RunArgs<T> *__restrict__ 
 }
 
 template <class T, int DIR, Recon RC, RSolver RS>
-__global__ void __launch_bounds__(BX * BY) kb_flux_m(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+__global__ void __launch_bounds__(BX * BY, (march_waves_v<T, RC>)) kb_flux_m(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
                                                  const int *__restrict__ nitem, const int cur) {
+  __shared__ T park[park_n<T, RC, false>];
   const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
     const Item m = uniform_item(item, it);
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][DIR];
-    flux_m_tile<T, DIR, RC, RS, false>(a, m.tile);
+    flux_m_tile<T, DIR, RC, RS, false>(a, m.tile, park);
   }
 }
 
