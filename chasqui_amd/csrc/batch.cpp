@@ -5,8 +5,8 @@
 //
 // One RK step is the same kernel sequence as a single context's fused step, each launch
 // covering every run: flux x1..x3, corner EMF, update, ghost fill + con2prim (+ fofc list),
-// then the fofc branch over the runs that flagged cells (compacted on the device), then the
-// control-block updates (per-run dt, t, cycle, primitive-set flip). No reduction spans runs,
+// then the fofc branch over the runs that flagged cells (compacted on the device), whose last launch
+// makes the control-block updates (per-run dt, t, cycle, primitive-set flip). No reduction spans runs,
 // so every run's result is bitwise the one it gets alone.
 //
 // The step is captured once in a hipGraph and replayed. Lists and the run count live in device
@@ -175,14 +175,25 @@ struct Batch final : BatchBase {
     const int n = int(b->runs.size());
     h_runs.resize(size_t(n));
     for (int r = 0; r < n; ++r) h_runs[r] = describe(b->runs[r]);
-    // the y/z march segment follows the march work of the whole batch per direction
-    for (int d = 1; d < 3; ++d) {
-      std::vector<fluxk::MarchShape> shapes;
-      for (int r = 0; r < n; ++r) {
+    // The y/z march segment follows the march work of the whole batch: all of it if the directions
+    // go in one launch (a batch with little of it, by the rule of a single mesh), else per direction.
+    std::vector<fluxk::MarchShape> shapes[3], all;   // [direction]
+    long long blocks = 0;
+    bool d3 = true;
+    for (int r = 0; r < n; ++r) {
+      if (h_runs[r].ndir == 2) d3 = false;
+      for (int d = 1; d < h_runs[r].ndir; ++d) {
         const FluxArgsT<T> &a = h_runs[r].flux[0][0][d];
-        if (d < h_runs[r].ndir) shapes.push_back(fluxk::march_shape(a.il, a.iu, a.jl, a.ju, a.kl, a.ku, d));
+        const fluxk::MarchShape m = fluxk::march_shape(a.il, a.iu, a.jl, a.ju, a.kl, a.ku, d);
+        shapes[d].push_back(m);
+        all.push_back(m);
+        blocks += m.rows * m.nd / 256;
       }
-      const int seg = fluxk::march_seg(shapes.data(), int(shapes.size()));
+    }
+    merge = !all.empty() && fluxk::merge_blocks(sizeof(T) == 4, false, Recon(b->recon), d3, blocks);
+    for (int d = 1; d < 3; ++d) {
+      const int seg = merge ? fluxk::joint_seg(all.data(), int(all.size()))
+                            : fluxk::march_seg(shapes[d].data(), int(shapes[d].size()));
       for (int r = 0; r < n; ++r)
         for (auto &row : h_runs[r].flux)
           for (auto &ws : row) ws[d].seg = seg;
@@ -237,8 +248,9 @@ struct Batch final : BatchBase {
 
   // The launches of a stage; classes that no run of the batch has (the y and z fluxes
   // of 1D runs, z of 2D, the corner EMF launch of 3D) are left out (present[], fixed when the step is enqueued or
-  // captured; a change re-captures the graph). The control launches between stages are merged:
-  // begin step + begin stage 1, end stage + begin next, end last stage + end step.
+  // captured; a change re-captures the graph). The control work between stages is merged: begin step +
+  // begin stage 1 in a launch, end stage + begin next and end last stage + end step in the fofc
+  // branch's last launch.
   int enqueue_stage(int s) {
     const Coef cf = rk_coef(b->nstage, s);
     const int last = s == b->nstage;
@@ -246,25 +258,30 @@ struct Batch final : BatchBase {
     const RSolver rs = RSolver(b->rsolver);
     hipStream_t st = b->stream;
     const int *g = b->grid;
+    if (merge) {
+      const ItemList fl[3] = {list(K_FLUX1), list(K_FLUX2), list(K_FLUX3)};
+      HIPCHK(launchb_flux_all(d_runs, fl, cf.cur, rc, rs, std::max({g[K_FLUX1], g[K_FLUX2], g[K_FLUX3]}), st));
+    }
     for (int d = 0; d < 3; ++d)
-      if (present[K_FLUX1 + d]) HIPCHK(launchb_flux(d_runs, list(K_FLUX1 + d), d, cf.cur, rc, rs, g[K_FLUX1 + d], st));
+      if (present[K_FLUX1 + d] && !merge) HIPCHK(launchb_flux(d_runs, list(K_FLUX1 + d), d, cf.cur, rc, rs, g[K_FLUX1 + d], st));
     if (present[K_CORNER]) HIPCHK(launchb_corner<T>(d_runs, list(K_CORNER), g[K_CORNER], st));
     HIPCHK(launchb_update<T>(d_runs, list(K_UPDATE), cf.out, cf.g0, cf.g1, cf.beta, g[K_UPDATE], st));
     HIPCHK(launchb_c2p<T>(d_runs, list(K_C2P), cf.out, last, g[K_C2P], st));
+    const int op = last ? CTRL_END_LAST : CTRL_TURN, arg = last ? 0 : s + 1 == b->nstage;
     // fofc branch of the runs that flagged cells: for batches of small runs, one block per run
     // in two launches; otherwise compacted over the flagged runs, one launch per class
     if (small_branch) {
       HIPCHK(launchb_repair_runs(d_runs, d_count, b->capacity, cf.cur, st));
-      HIPCHK(launchb_fofc_runs<T>(d_runs, d_count, b->capacity, cf.out, cf.g0, cf.g1, cf.beta, last, st));
+      HIPCHK(launchb_fofc_runs<T>(d_runs, d_count, b->capacity, cf.out, cf.g0, cf.g1, cf.beta, last, op, arg,
+                                  d_live, st));
     } else {
       HIPCHK(launchb_fofc_scan<T>(d_runs, d_count, cond(), st));
       HIPCHK(launchb_repair(d_runs, cond(), cf.cur, g[G_REPAIR], st));
       if (present[K_CORNER]) HIPCHK(launchb_corner_cond<T>(d_runs, cond(), g[G_REPAIR], st));
       HIPCHK(launchb_update_cond<T>(d_runs, cond(), cf.out, cf.g0, cf.g1, cf.beta, g[G_COND], st));
-      HIPCHK(launchb_c2p_cond<T>(d_runs, cond(), cf.out, last, g[G_COND], st));
+      HIPCHK(launchb_c2p_cond<T>(d_runs, d_count, cond(), cf.out, last, op, arg, d_live, g[G_COND], st));
     }
-    if (last) return ctrl(CTRL_END_LAST, 0);
-    return ctrl(CTRL_TURN, s + 1 == b->nstage);
+    return CHQ_OK;
   }
 
   int enqueue_step() override {
@@ -279,6 +296,7 @@ struct Batch final : BatchBase {
 
   bool present[K_NLIST]{};
   bool small_branch = false;
+  bool merge = false;   // the face fluxes of all directions in one launch (set by rebuild)
   unsigned captured_present = ~0u;
   // the runs' fofc branch fits one block each: at most SMALL_BRANCH_TILES tiles of re-update,
   // ghost fill and con2prim per run (a few thousand cells), where launches cost more than the
@@ -296,7 +314,7 @@ struct Batch final : BatchBase {
   unsigned present_mask() const {
     unsigned m = 0;
     for (int k = 0; k < K_NLIST; ++k) m |= (h_count[1 + k] > 0 ? 1u : 0u) << k;
-    return m | (small_runs() ? 1u << K_NLIST : 0u);
+    return m | (small_runs() ? 1u << K_NLIST : 0u) | (merge ? 2u << K_NLIST : 0u);
   }
 
   // one timed launch of class q with grid gsz, in the stage-1 configuration (input buffer 0,

@@ -61,6 +61,10 @@ hipError_t launchb_flux(const RunArgs<double> *R, ItemList L, int dir, int cur, 
   return fluxk::launchb_flux_t<double>(R, L, dir, cur, rc, rs, grid, s);
 }
 
+hipError_t launchb_flux_all(const RunArgs<double> *R, const ItemList L[3], int cur, Recon rc, RSolver rs, int grid, hipStream_t s) {
+  return fluxk::launchb_flux_all_t<double>(R, L, cur, rc, rs, grid, s);
+}
+
 hipError_t launchb_repair(const RunArgs<double> *R, CondList C, int cur, int grid, hipStream_t s) {
   return fluxk::launchb_repair_t<double>(R, C, cur, grid, s);
 }

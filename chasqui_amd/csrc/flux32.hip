@@ -31,6 +31,10 @@ hipError_t launchb_flux(const RunArgs<float> *R, ItemList L, int dir, int cur, R
   return fluxk::launchb_flux_t<float>(R, L, dir, cur, rc, rs, grid, s);
 }
 
+hipError_t launchb_flux_all(const RunArgs<float> *R, const ItemList L[3], int cur, Recon rc, RSolver rs, int grid, hipStream_t s) {
+  return fluxk::launchb_flux_all_t<float>(R, L, cur, rc, rs, grid, s);
+}
+
 hipError_t launchb_repair(const RunArgs<float> *R, CondList C, int cur, int grid, hipStream_t s) {
   return fluxk::launchb_repair_t<float>(R, C, cur, grid, s);
 }

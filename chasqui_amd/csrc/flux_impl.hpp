@@ -647,6 +647,32 @@ __global__ void __launch_bounds__(BX * BY, (march_waves_v<T, RC>)) kb_flux_m(con
   }
 }
 
+// All directions of a batch with little work in one launch, in the order of k_flux_all.
+template <class T, Recon RC, RSolver RS>
+__global__ void __launch_bounds__(256, (march_waves_v<T, RC>)) kb_flux_all(
+    const RunArgs<T> *__restrict__ R, const Item *__restrict__ item0, const Item *__restrict__ item1,
+    const Item *__restrict__ item2, const int *__restrict__ n0, const int *__restrict__ n1, const int *__restrict__ n2,
+    const int cur) {
+  __shared__ T park[park_n<T, RC, false>];
+  const int ny = *n1, nz = *n2, n = ny + nz + *n0;
+  for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
+    const int dir = it < ny ? 1 : it < ny + nz ? 2 : 0;
+    const Item m = dir == 1 ? uniform_item(item1, it) : dir == 2 ? uniform_item(item2, it - ny)
+                                                                 : uniform_item(item0, it - ny - nz);
+    const Ctrl *ctl = R[m.run].ctrl;
+    if (!ctl->active) continue;
+    const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][dir];
+    if (dir == 1) flux_m_tile<T, 1, RC, RS, false>(a, m.tile, park);
+    else if (dir == 2) flux_m_tile<T, 2, RC, RS, false>(a, m.tile, park);
+    else {
+      int nseg, nwaves;
+      x_shape(a, fpw_v<RC>, nseg, nwaves);
+      const int wave = m.tile * 4 + int(threadIdx.x >> 6);
+      if (wave < nwaves) flux_x_wave<T, RC, RS, false>(a, nseg, wave);
+    }
+  }
+}
+
 // fofc repair of the flagged runs (compacted list, tiles of 256 (cell, face) entries)
 // entry t of run r's repair: face `side` of direction `dir` of listed cell t / (2 ndir)
 template <class T>
@@ -718,6 +744,26 @@ hipError_t launchb_flux_t(const RunArgs<T> *R, ItemList L, int dir, int cur, Rec
   if (dir == 0) return gob_flux_rc<T, 0>(R, L, cur, rc, rs, grid, s);
   if (dir == 1) return gob_flux_rc<T, 1>(R, L, cur, rc, rs, grid, s);
   return gob_flux_rc<T, 2>(R, L, cur, rc, rs, grid, s);
+}
+
+template <class T, Recon RC>
+hipError_t gob_flux_all(const RunArgs<T> *R, const ItemList L[3], int cur, RSolver rs, int grid, hipStream_t s) {
+  const dim3 g(grid), b(256);
+  if (rs == RSolver::hlld) hipLaunchKernelGGL((kb_flux_all<T, RC, RSolver::hlld>), g, b, 0, s, R, L[0].item, L[1].item, L[2].item, L[0].n, L[1].n, L[2].n, cur);
+  else if (rs == RSolver::lhlld) hipLaunchKernelGGL((kb_flux_all<T, RC, RSolver::lhlld>), g, b, 0, s, R, L[0].item, L[1].item, L[2].item, L[0].n, L[1].n, L[2].n, cur);
+  else hipLaunchKernelGGL((kb_flux_all<T, RC, RSolver::hlle>), g, b, 0, s, R, L[0].item, L[1].item, L[2].item, L[0].n, L[1].n, L[2].n, cur);
+  return hipGetLastError();
+}
+
+template <class T>
+hipError_t launchb_flux_all_t(const RunArgs<T> *R, const ItemList L[3], int cur, Recon rc, RSolver rs, int grid, hipStream_t s) {
+  switch (rc) {
+    case Recon::dc: return gob_flux_all<T, Recon::dc>(R, L, cur, rs, grid, s);
+    case Recon::plm: return gob_flux_all<T, Recon::plm>(R, L, cur, rs, grid, s);
+    case Recon::ppm: return gob_flux_all<T, Recon::ppm>(R, L, cur, rs, grid, s);
+    case Recon::ppmx: return gob_flux_all<T, Recon::ppmx>(R, L, cur, rs, grid, s);
+    default: return gob_flux_all<T, Recon::wenoz>(R, L, cur, rs, grid, s);
+  }
 }
 
 template <class T>

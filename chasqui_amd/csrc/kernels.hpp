@@ -295,6 +295,14 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
 //   FP32   PPM    160^3 (33010) 2.45 -> 2.36, 192^3 (56748) no gain over a whole run, 256^3 8.59 -> 8.72;
 //                 1000x1024 0.440 -> 0.427, 2000^2 1.63 -> 1.65
 //          WENO-Z 256^3 (133648) 9.62 -> 9.41, 2000^2 (15648) 1.78 -> 1.76
+// A batch counts the march blocks of all its runs (64 small mixed runs 28.4 -> 26.6 ms per 100 steps).
+inline bool merge_blocks(bool fp32, bool charac, Recon rc, bool d3, long long blocks) {
+  const bool weno = rc == Recon::wenoz;
+  if (fp32) return weno ? (d3 || blocks <= 16000) : blocks <= (d3 ? 40000 : 8000);
+  if (charac) return d3 && blocks <= 4500;
+  if (weno) return blocks <= (d3 ? 7500 : 1500);
+  return blocks <= (d3 ? (rc == Recon::ppmx ? 18000 : 34000) : 4500);
+}
 template <class T>
 inline bool flux_merge(const FluxArgsT<T> *a, int ndir, Recon rc, bool entropy) {
   if (ndir < 2 || (entropy && !a[0].charac)) return false;
@@ -303,30 +311,29 @@ inline bool flux_merge(const FluxArgsT<T> *a, int ndir, Recon rc, bool entropy) 
     const MarchShape m = march_shape(a[d].il, a[d].iu, a[d].jl, a[d].ju, a[d].kl, a[d].ku, d);
     blocks += m.rows * m.nd / 256;
   }
-  const bool weno = rc == Recon::wenoz, d3 = ndir == 3;
-  if (sizeof(T) == 4) return weno ? (d3 || blocks <= 16000) : blocks <= (d3 ? 40000 : 8000);
-  if (a[0].charac) return d3 && blocks <= 4500;
-  if (weno) return blocks <= (d3 ? 7500 : 1500);
-  return blocks <= (d3 ? (rc == Recon::ppmx ? 18000 : 34000) : 4500);
+  return merge_blocks(sizeof(T) == 4, a[0].charac, rc, ndir == 3, blocks);
 }
 // The march segment of a joint launch: the candidate of least (s + 1.5) (0.5 + m), m the march
 // blocks per CU. Blocks of all lengths share a CU here, so the work term has no steps at whole
 // blocks per CU as march_seg's has; fitted to sweeps over the sizes above (1.2% from the best
 // candidate on average).
-template <class T>
-inline void joint_seg(FluxArgsT<T> *a, int ndir) {
+inline int joint_seg(const MarchShape *sh, int n) {
   static constexpr int cand[] = {1, 2, 3, 4, 6, 8, 12, 16, 24};
   int best = 1;
   double least = 1e300;
   for (const int s : cand) {
     double blocks = 0.0;
-    for (int d = 1; d < ndir; ++d) {
-      const MarchShape m = march_shape(a[d].il, a[d].iu, a[d].jl, a[d].ju, a[d].kl, a[d].ku, d);
-      blocks += double(m.rows) * ((m.nd + s - 1) / s) / 256.0;
-    }
+    for (int q = 0; q < n; ++q) blocks += double(sh[q].rows) * ((sh[q].nd + s - 1) / s) / 256.0;
     const double cost = (s + 1.5) * (0.5 + blocks / 256.0);
     if (cost < least) { least = cost; best = s; }
   }
+  return best;
+}
+template <class T>
+inline void joint_seg(FluxArgsT<T> *a, int ndir) {
+  MarchShape sh[2];
+  for (int d = 1; d < ndir; ++d) sh[d - 1] = march_shape(a[d].il, a[d].iu, a[d].jl, a[d].ju, a[d].kl, a[d].ku, d);
+  const int best = joint_seg(sh, ndir - 1);
   for (int d = 1; d < ndir; ++d) a[d].seg = best;
 }
 
@@ -360,11 +367,12 @@ struct RunArgs {
 enum : int { CL_REPAIR = 0, CL_CORNER, CL_UPDATE, CL_C2P, CL_N };
 struct CondList {
   int cap;             // capacity in runs
-  int *base;           // [0] = number of flagged runs, then run[cap], then pre[CL_N][cap + 1]
+  int *base;           // [0] = number of flagged runs, then run[cap], then pre[CL_N][cap + 1], then done()
   __host__ __device__ int *nrun() const { return base; }
   __host__ __device__ int *run() const { return base + 1; }
   __host__ __device__ int *pre(int cls) const { return base + 1 + cap + cls * (cap + 1); }
-  static size_t ints(int cap) { return size_t(1) + cap + size_t(CL_N) * (cap + 1); }
+  __host__ __device__ int *done() const { return pre(CL_N); }   // finished blocks of the last launch (0 between)
+  static size_t ints(int cap) { return size_t(2) + cap + size_t(CL_N) * (cap + 1); }
 };
 
 // launches (defined in stage.hip / flux.hip / flux32.hip)
@@ -470,21 +478,28 @@ hipError_t launch_ctrl_begin_stage(Ctrl *c, int reset_slots, hipStream_t s);
 // launch arguments, everything per run comes from the RunArgs table
 hipError_t launchb_flux(const RunArgs<double> *R, ItemList L, int dir, int cur, Recon rc, RSolver rs, int grid, hipStream_t s);
 hipError_t launchb_flux(const RunArgs<float> *R, ItemList L, int dir, int cur, Recon rc, RSolver rs, int grid, hipStream_t s);
+// the lists of all directions in one launch (the batch's march work is below flux_merge's limits)
+hipError_t launchb_flux_all(const RunArgs<double> *R, const ItemList L[3], int cur, Recon rc, RSolver rs, int grid, hipStream_t s);
+hipError_t launchb_flux_all(const RunArgs<float> *R, const ItemList L[3], int cur, Recon rc, RSolver rs, int grid, hipStream_t s);
 hipError_t launchb_repair(const RunArgs<double> *R, CondList C, int cur, int grid, hipStream_t s);
 hipError_t launchb_repair(const RunArgs<float> *R, CondList C, int cur, int grid, hipStream_t s);
 // the fofc branch of a batch of small runs: one block per run (cap blocks), the repair, then the
-// edge EMFs, re-update, boundaries and con2prim of the run
+// edge EMFs, re-update, boundaries and con2prim of the run, and the stage's control turn (launchb_ctrl's
+// op, arg and live)
 hipError_t launchb_repair_runs(const RunArgs<double> *R, const int *nruns, int cap, int cur, hipStream_t s);
 hipError_t launchb_repair_runs(const RunArgs<float> *R, const int *nruns, int cap, int cur, hipStream_t s);
 template <class T> hipError_t launchb_fofc_runs(const RunArgs<T> *R, const int *nruns, int cap, int out, double g0,
-                                                double g1, double beta, int last, hipStream_t s);
+                                                double g1, double beta, int last, int op, int arg, int *live,
+                                                hipStream_t s);
 template <class T> hipError_t launchb_corner(const RunArgs<T> *R, ItemList L, int grid, hipStream_t s);
 template <class T> hipError_t launchb_update(const RunArgs<T> *R, ItemList L, int out, double g0, double g1, double beta, int grid, hipStream_t s);
 template <class T> hipError_t launchb_c2p(const RunArgs<T> *R, ItemList L, int buf, int last, int grid, hipStream_t s);
 template <class T> hipError_t launchb_fofc_scan(const RunArgs<T> *R, const int *nruns, CondList C, hipStream_t s);
 template <class T> hipError_t launchb_corner_cond(const RunArgs<T> *R, CondList C, int grid, hipStream_t s);
 template <class T> hipError_t launchb_update_cond(const RunArgs<T> *R, CondList C, int out, double g0, double g1, double beta, int grid, hipStream_t s);
-template <class T> hipError_t launchb_c2p_cond(const RunArgs<T> *R, CondList C, int buf, int last, int grid, hipStream_t s);
+// ... which ends the stage of every run with the control work op, arg, live (launchb_ctrl)
+template <class T> hipError_t launchb_c2p_cond(const RunArgs<T> *R, const int *nruns, CondList C, int buf, int last, int op,
+                                               int arg, int *live, int grid, hipStream_t s);
 // control-block step of every run (one thread per table slot, `cap` slots); the end of a step
 // also writes live[r] = run r has not reached tlim / nlim
 template <class T> hipError_t launchb_ctrl(const RunArgs<T> *R, const int *nruns, int cap, int op, int arg, int *live, hipStream_t s);
