@@ -216,6 +216,7 @@ int chq_create(const chq_mesh_desc *m, const chq_config *cfg, chq_ctx **out) {
   c->x1min = m->x1min; c->x2min = m->x2min; c->x3min = m->x3min;
   c->eos.gamma = cfg->gamma;
   c->eos.gm1 = cfg->gamma - 1.0;
+  c->eos.igm1 = 1.0 / c->eos.gm1;
   c->eos.dfloor = cfg->dfloor;
   c->eos.pfloor = cfg->pfloor;
   c->eos.dual_energy = cfg->dual_energy;

@@ -34,6 +34,7 @@ struct Geom {
 
 struct Eos {
   double gamma, gm1, dfloor, pfloor;
+  double igm1;      // 1 / gm1
   int dual_energy;
   double de_eta;
 };

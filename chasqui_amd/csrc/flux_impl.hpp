@@ -57,7 +57,7 @@ __device__ __forceinline__ void solve_face(const FluxArgsT<T> &a, long long c, l
                                            const T *Rs_, T f[NFLX]) {
   using V = Rsv<T>;
   const Geom &g = a.g;
-  const T gam = T(a.eos.gamma), gm1 = T(a.eos.gm1);
+  const T gam = T(a.eos.gamma), gm1 = T(a.eos.gm1), igm1 = T(a.eos.igm1);
   const long long cs = g.cstride;
   constexpr int IU = IVX + DIR, IV = IVX + (DIR + 1) % 3, IW = IVX + (DIR + 2) % 3;
   St<T> L{Ls[0], Ls[1], Ls[2], Ls[3], Ls[4], Ls[5], Ls[6]};
@@ -71,7 +71,7 @@ __device__ __forceinline__ void solve_face(const FluxArgsT<T> &a, long long c, l
     R.u = um - ud;
   }
   if constexpr (RS == RSolver::hlld) {
-    V::template hlld<false>(L, R, bn, gam, gm1, f);
+    V::template hlld<false>(L, R, bn, gam, gm1, igm1, f);
   } else if constexpr (RS == RSolver::lhlld) {                     // physics.hpp:182-211
     constexpr int t1 = (DIR + 1) % 3, t2 = (DIR + 2) % 3;
     const T *wu = a.w + IU * cs, *wv = a.w + IV * cs, *ww = a.w + IW * cs;
@@ -96,7 +96,7 @@ __device__ __forceinline__ void solve_face(const FluxArgsT<T> &a, long long c, l
     const T theta = r2 * r2;
     const T chi = vmin(T(1), vmax(V::cflow(L, bn), V::cflow(R, bn)) / cfm);
     const T phi = (a.lhlld_phi >= 0.0) ? T(a.lhlld_phi) : chi * (T(2) - chi);
-    V::template hlld<true>(L, R, bn, gam, gm1, f, theta, phi);
+    V::template hlld<true>(L, R, bn, gam, gm1, igm1, f, theta, phi);
   } else {
     V::hlle(L, R, bn, gam, gm1, f);
   }
