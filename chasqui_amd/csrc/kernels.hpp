@@ -284,24 +284,24 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
 // Whether the face fluxes of all directions go in one launch (k_flux_all, k_fluxc_all). One launch
 // saves the others' dispatch and tails and lets the x blocks fill the SIMDs that a small march
 // leaves idle; but the x waves then run at the march's occupancy (two waves per SIMD in FP64
-// instead of four, three instead of eight in FP32), which costs more once each launch fills the
+// instead of four, four instead of eight in FP32), which costs more once each launch fills the
 // device by itself. The limits are on the march blocks at one face per thread, both sides measured
 // (ms per RK3 step, separate -> one launch):
-//   FP64   PPM    64x56x45 (1378 blocks) 0.336 -> 0.269, 160^3 (33010) 3.93 -> 3.81, 192^3 6.28 -> 6.36;
-//                 512^2 PPMX (1030) 0.300 -> 0.264, 1000x1024 (4011) 0.723 -> 0.715, 2000^2 2.58 -> 2.64
-//          PPMX   128^3 (17032) 2.50 -> 2.48, 160^3 4.47 -> 4.60
-//          WENO-Z 512^2 (1030) 0.419 -> 0.389, 750^2 0.726 -> 0.735; 96^3 (7278) 1.64 -> 1.61, 128^3 3.40 -> 3.48
-//          characteristic PPMX 80x72x64 (3083) 1.087 -> 1.009, 96^3 2.12 -> 2.18; 500^2 0.378 -> 0.382
-//   FP32   PPM    160^3 (33010) 2.45 -> 2.36, 192^3 (56748) no gain over a whole run, 256^3 8.59 -> 8.72;
-//                 1000x1024 0.440 -> 0.427, 2000^2 1.63 -> 1.65
-//          WENO-Z 256^3 (133648) 9.62 -> 9.41, 2000^2 (15648) 1.78 -> 1.76
+//   FP64   PPM    64x56x45 (1378 blocks) 0.336 -> 0.269; the whole pass at 128^3 (17032) -1.3%, 160^3 -1.2%, 208^3
+//                 (72031) -0.6%, 256^3 (133648) +1.6%; 800^2 (2519) -2.8%, 1000^2 (3929) -0.3%, 1200^2 +0.4%; PLM and
+//                 PPMX alike (PPMX 144^3 -3.4%, 208^3 -0.2%)
+//          WENO-Z 64^3 -15%, 144^3 (24145) -4.3%, 192^3 (56748) -1.1%, 224^3 (89778) +1.4%; 400^2 -8%, 800^2
+//                 -4.2%, 1000^2 -0.3%
+//          characteristic PPMX 64^3 (2212) -11%, 80x72x64 (3083) 1.087 -> 1.009, 96^3 (7278) +1.4%; 500^2 0.378 -> 0.382
+//   FP32   PPM    144^3 (24145) -3.5%, 192^3 (56748) -2.2% for a wave but 30 steps of a blast +0.6%, 240^3 -0.2%, PPMX
+//                 there +1.3%; 1300^2 (6616) -1.9%, 1600^2 +0.6%; PLM 192^3 +0.3%
+//          WENO-Z 192^3 -2.1%, 256^3 (133648) 9.62 -> 9.41; 1600^2 (10022) -2%, 2000^2 (15648) 1.78 -> 1.76
 // A batch counts the march blocks of all its runs (64 small mixed runs 28.4 -> 26.6 ms per 100 steps).
 inline bool merge_blocks(bool fp32, bool charac, Recon rc, bool d3, long long blocks) {
   const bool weno = rc == Recon::wenoz;
   if (fp32) return weno ? (d3 || blocks <= 16000) : blocks <= (d3 ? 40000 : 8000);
   if (charac) return d3 && blocks <= 4500;
-  if (weno) return blocks <= (d3 ? 7500 : 1500);
-  return blocks <= (d3 ? (rc == Recon::ppmx ? 18000 : 34000) : 4500);
+  return blocks <= (d3 ? (weno ? 65000 : 75000) : 4500);
 }
 template <class T>
 inline bool flux_merge(const FluxArgsT<T> *a, int ndir, Recon rc, bool entropy) {
