@@ -10,7 +10,7 @@
 // cell is done once and hands its two half-states to its two faces:
 //   * x faces: lane = cell, the window arrives through DPP whole-wave shifts;
 //   * y and z faces: lane = i, each thread marches a.seg faces along the direction with the
-//     raw window in registers.
+//     raw window's cell in registers and its neighbours in LDS.
 // Sums keep the reference's order (ascending variable index for the projection, ascending
 // wave index for the map back); the structurally zero matrix entries are left out. The
 // accumulators start at +0 as in the reference and an added product with a zero entry can
@@ -98,8 +98,16 @@ __device__ __forceinline__ void eigen_of(double d, double p, double by, double b
 }
 
 // characteristic variable KK of one stencil point: sum_n L[KK][n] q[n], ascending n, from +0
-template <int KK>
-__device__ __forceinline__ double project(const Eig &E, const double *q) {
+// The 7 or 8 variables of one window cell in LDS, a thread's entries SP apart.
+struct Parked {
+  static constexpr int SP = BX * BY;
+  double *p;
+  __device__ __forceinline__ double operator[](int n) const { return p[n * SP]; }
+  __device__ __forceinline__ void set(int n, double v) const { p[n * SP] = v; }
+};
+
+template <int KK, class Q>
+__device__ __forceinline__ double project(const Eig &E, const Q &q) {
   double acc = 0.0;
   if constexpr (KK == 0) {
     acc += E.l0[1] * q[1]; acc += E.l0[2] * q[2]; acc += E.l0[3] * q[3];
@@ -139,39 +147,42 @@ __device__ __forceinline__ void map_back(const Eig &E, double ch, double out[7])
   }
 }
 
-template <Recon RC, int KK>
-__device__ __forceinline__ void wave_step(const Eig &E, const double (&r)[5][8], double Lf[7], double Rf[7]) {
+template <Recon RC, int KK, class Q>
+__device__ __forceinline__ void wave_step(const Eig &E, const Q &q0, const Q &q1, const double (&q2)[8], const Q &q3,
+                                          const Q &q4, double Lf[7], double Rf[7]) {
   constexpr bool W = wide_v<RC>;
-  const double c1 = project<KK>(E, r[1]), c2 = project<KK>(E, r[2]), c3 = project<KK>(E, r[3]);
-  const double c0 = W ? project<KK>(E, r[0]) : c1;
-  const double c4 = W ? project<KK>(E, r[4]) : c3;
+  const double c1 = project<KK>(E, q1), c2 = project<KK>(E, q2), c3 = project<KK>(E, q3);
+  const double c0 = W ? project<KK>(E, q0) : c1;
+  const double c4 = W ? project<KK>(E, q4) : c3;
   double lo, hi;
   cell_halves<double, RC>(c0, c1, c2, c3, c4, lo, hi);
   map_back<KK>(E, hi, Lf);
   map_back<KK>(E, lo, Rf);
+  // (a parked window is read again for the next wave instead of held in registers)
+  if constexpr (std::is_same<Q, Parked>::value) asm volatile("" ::: "memory");
 }
 
-// Half-states of cell c (window r[0..4] = raw primitives of c-2..c+2, slots 0..6 in the
+// Half-states of cell c (q0..q4 = raw primitives of c-2..c+2, slots 0..6 in the
 // rotated frame) in the characteristic variables of c; bxn = cell-centred normal field of c.
 // Lf = right-edge value of c (left state of face c+1/2), Rf = left-edge value (right state of
-// face c-1/2). Narrow methods read r[1..3] only.
-template <Recon RC>
-__device__ __forceinline__ void charac_cell(const double (&r)[5][8], double bxn, double gamma, double Lf[7],
-                                            double Rf[7]) {
+// face c-1/2). Narrow methods read q1..q3 only.
+template <Recon RC, class Q>
+__device__ __forceinline__ void charac_cell(const Q &q0, const Q &q1, const double (&q2)[8], const Q &q3, const Q &q4,
+                                            double bxn, double gamma, double Lf[7], double Rf[7]) {
   Eig E;
-  eigen_of(r[2][0], r[2][4], r[2][5], r[2][6], bxn, gamma, E);
+  eigen_of(q2[0], q2[4], q2[5], q2[6], bxn, gamma, E);
 #pragma unroll
   for (int n = 0; n < 7; ++n) {
     Lf[n] = 0.0;
     Rf[n] = 0.0;
   }
-  wave_step<RC, 0>(E, r, Lf, Rf);
-  wave_step<RC, 1>(E, r, Lf, Rf);
-  wave_step<RC, 2>(E, r, Lf, Rf);
-  wave_step<RC, 3>(E, r, Lf, Rf);
-  wave_step<RC, 4>(E, r, Lf, Rf);
-  wave_step<RC, 5>(E, r, Lf, Rf);
-  wave_step<RC, 6>(E, r, Lf, Rf);
+  wave_step<RC, 0>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 1>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 2>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 3>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 4>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 5>(E, q0, q1, q2, q3, q4, Lf, Rf);
+  wave_step<RC, 6>(E, q0, q1, q2, q3, q4, Lf, Rf);
 }
 
 // ---------------------------------------------------------------- x faces: lane = cell
@@ -206,7 +217,7 @@ __device__ __forceinline__ void fluxc_x_wave(const FluxArgsT<double> &a, const i
   }
   const double bxn = a.bcc[row0 + ci];   // component 0 = the x1 (normal) field
   double Lf[NV], Rf[NV];
-  charac_cell<RC>(r, bxn, a.eos.gamma, Lf, Rf);
+  charac_cell<RC>(r[0], r[1], r[2], r[3], r[4], bxn, a.eos.gamma, Lf, Rf);
   if constexpr (ENT) cell_halves<double, RC>(r[0][7], r[1][7], r[2][7], r[3][7], r[4][7], Rf[7], Lf[7]);
   double fco = 0.0;
   if constexpr (W) {
@@ -234,8 +245,13 @@ __global__ void __launch_bounds__(256) k_fluxc_x(const FluxArgsT<double> a, cons
 }
 
 // ---------------------------------------------------------------- y/z faces: register march
+// The window's neighbours (four cells) and the left state of the next face stay in LDS, 70 or 80 KB a
+// block, two blocks per CU: with the eigenvectors beside them in registers the march took 256 VGPRs and
+// up to 76 accumulation registers, one wave per SIMD; now 212 to 254, two. ms per pass of 6 steps, PPMX,
+// LHLLD, dual energy: 64^3 5.48 -> 4.69, 80^3 9.87 -> 8.37, 96^3 15.4 -> 14.3, 112^3 22.4 -> 20.9.
+template <bool ENT> constexpr int cpark_n = 5 * (ENT ? 8 : 7) * BX * BY;
 template <int DIR, Recon RC, RSolver RS, bool ENT>
-__device__ __forceinline__ void fluxc_m_tile(const FluxArgsT<double> &a, const int bx) {
+__device__ __forceinline__ void fluxc_m_tile(const FluxArgsT<double> &a, const int bx, double *park) {
   constexpr int NV = ENT ? 8 : 7;
   constexpr bool W = wide_v<RC>;
   const Geom &g = a.g;
@@ -252,73 +268,91 @@ __device__ __forceinline__ void fluxc_m_tile(const FluxArgsT<double> &a, const i
   const double *src[NV];
   var_ptrs<double, DIR, NV>(a, src);
   const double *bnc = a.bcc + DIR * g.cstride;   // cell-centred normal field
-  // raw window of the cell being finished, c: r[m] = q_{c-2+m} (narrow methods: m = 1..3)
-  double r[5][8];
+  // raw window of the cell being finished, c: q_{c-2} .. q_{c+2} (narrow methods: c-1 .. c+1); the cell
+  // itself in registers, the others and the left state of face c parked
+  double *const pk = park + int(threadIdx.y) * BX + int(threadIdx.x);
+  constexpr int ROW = NV * Parked::SP;
+  Parked q0{pk}, q1{pk + ROW}, q3{pk + 2 * ROW}, q4{pk + 3 * ROW};
+  const Parked lp{pk + 4 * ROW};
+  double q2[8];
   int c = F0 - 1;
   {
     const long long cc = base + (long long)c * sd;
 #pragma unroll
     for (int n = 0; n < NV; ++n) {
-      r[1][n] = src[n][cc - sd];
-      r[2][n] = src[n][cc];
-      r[3][n] = src[n][cc + sd];
-      r[0][n] = W ? src[n][cc - 2 * sd] : r[1][n];
-      r[4][n] = W ? src[n][cc + 2 * sd] : r[3][n];
+      q2[n] = src[n][cc];
+      q1.set(n, src[n][cc - sd]);
+      q3.set(n, src[n][cc + sd]);
+      if constexpr (W) {
+        q0.set(n, src[n][cc - 2 * sd]);
+        q4.set(n, src[n][cc + 2 * sd]);
+      }
     }
   }
-  double Lprev[NV];
   for (; c <= F1; ++c) {
     const long long cc = base + (long long)c * sd;
     double Lf[NV], Rf[NV];
-    charac_cell<RC>(r, bnc[cc], a.eos.gamma, Lf, Rf);
-    if constexpr (ENT) cell_halves<double, RC>(r[0][7], r[1][7], r[2][7], r[3][7], r[4][7], Rf[7], Lf[7]);
+    charac_cell<RC>(q0, q1, q2, q3, q4, bnc[cc], a.eos.gamma, Lf, Rf);
+    if constexpr (ENT)
+      cell_halves<double, RC>(W ? q0[7] : q1[7], q1[7], q2[7], q3[7], W ? q4[7] : q3[7], Rf[7], Lf[7]);
     double fco = 0.0;
     if constexpr (W) {
-      if (a.flatten) fco = Rec<double>::flat(r[0][4], r[1][4], r[2][4], r[3][4], r[4][4], r[1][1], r[3][1]);
+      if (a.flatten) fco = Rec<double>::flat(q0[4], q1[4], q2[4], q3[4], q4[4], q1[1], q3[1]);
     }
     double qc[NV];
 #pragma unroll
-    for (int n = 0; n < NV; ++n) qc[n] = r[2][n];
+    for (int n = 0; n < NV; ++n) qc[n] = q2[n];
     finish_cell<double, NV>(Lf, Rf, qc, fco, W && a.flatten, a.eos.dfloor, a.eos.pfloor);
-    if (c >= F0) solve_store<double, DIR, RS, ENT, NV>(a, cc, sd, Lprev, Rf);   // face c
+    double Lprev[NV];
 #pragma unroll
-    for (int n = 0; n < NV; ++n) Lprev[n] = Lf[n];
-    if (c < F1) {   // slide the window by one cell
+    for (int n = 0; n < NV; ++n) {
+      Lprev[n] = lp[n];
+      lp.set(n, Lf[n]);
+    }
+    asm volatile("" ::: "memory");
+    double nx[NV];   // on its way while the face is solved
+    if (c < F1) {
+#pragma unroll
+      for (int n = 0; n < NV; ++n) nx[n] = src[n][cc + (W ? 3 : 2) * sd];
+    }
+    if (c >= F0) solve_store<double, DIR, RS, ENT, NV>(a, cc, sd, Lprev, Rf);   // face c
+    if (c < F1) {   // slide the window by one cell: its rows change places, none is copied
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
-        if constexpr (W) {
-          r[0][n] = r[1][n];
-          r[1][n] = r[2][n];
-          r[2][n] = r[3][n];
-          r[3][n] = r[4][n];
-          r[4][n] = src[n][cc + 3 * sd];
-        } else {
-          r[1][n] = r[2][n];
-          r[2][n] = r[3][n];
-          r[3][n] = src[n][cc + 2 * sd];
-          r[0][n] = r[1][n];
-          r[4][n] = r[3][n];
-        }
+        const double up = q3[n];
+        (W ? q0 : q1).set(n, q2[n]);
+        q3.set(n, nx[n]);
+        q2[n] = up;
+      }
+      if constexpr (W) {
+        Parked t = q0;
+        q0 = q1;
+        q1 = t;
+        t = q3;
+        q3 = q4;
+        q4 = t;
       }
     }
   }
 }
 
 template <int DIR, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(BX * BY) k_fluxc_m(const FluxArgsT<double> a) {
+__global__ void __launch_bounds__(BX * BY, 2) k_fluxc_m(const FluxArgsT<double> a) {
+  __shared__ double park[cpark_n<ENT>];
   if (!a.ctrl->active) return;
-  fluxc_m_tile<DIR, RC, RS, ENT>(a, int(blockIdx.x));
+  fluxc_m_tile<DIR, RC, RS, ENT>(a, int(blockIdx.x), park);
 }
 
 // all directions of a small mesh in one launch (as k_flux_all)
 template <Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(256) k_fluxc_all(const FluxArgsT<double> a0, const FluxArgsT<double> a1,
+__global__ void __launch_bounds__(256, 2) k_fluxc_all(const FluxArgsT<double> a0, const FluxArgsT<double> a1,
                                                    const FluxArgsT<double> a2, const int nseg, const int nwaves,
                                                    const int nby, const int nbz) {
+  __shared__ double park[cpark_n<ENT>];
   if (!a0.ctrl->active) return;
   const int b = int(blockIdx.x);
-  if (b < nby) fluxc_m_tile<1, RC, RS, ENT>(a1, b);
-  else if (b < nby + nbz) fluxc_m_tile<2, RC, RS, ENT>(a2, b - nby);
+  if (b < nby) fluxc_m_tile<1, RC, RS, ENT>(a1, b, park);
+  else if (b < nby + nbz) fluxc_m_tile<2, RC, RS, ENT>(a2, b - nby, park);
   else {
     const int wave = (b - nby - nbz) * 4 + int(threadIdx.x >> 6);
     if (wave < nwaves) fluxc_x_wave<RC, RS, ENT>(a0, nseg, wave);
