@@ -292,7 +292,8 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
 //                 PPMX alike (PPMX 144^3 -3.4%, 208^3 -0.2%)
 //          WENO-Z 64^3 -15%, 144^3 (24145) -4.3%, 192^3 (56748) -1.1%, 224^3 (89778) +1.4%; 400^2 -8%, 800^2
 //                 -4.2%, 1000^2 -0.3%
-//          characteristic PPMX 64^3 (2212) -11%, 80x72x64 (3083) 1.087 -> 1.009, 96^3 (7278) +1.4%; 500^2 0.378 -> 0.382
+//          characteristic PPMX (x kernel and march both at two waves): 80x72x64 (3083) 1.087 -> 1.009, 96^3 (7278)
+//                 -8%, 112^3 -4%, 144^3 (24145) -7%; 200^2 -16%, 500^2 -11%: always
 //   FP32   PPM    144^3 (24145) -3.5%, 192^3 (56748) -2.2% for a wave but 30 steps of a blast +0.6%, 240^3 -0.2%, PPMX
 //                 there +1.3%; 1300^2 (6616) -1.9%, 1600^2 +0.6%; PLM 192^3 +0.3%
 //          WENO-Z 192^3 -2.1%, 256^3 (133648) 9.62 -> 9.41; 1600^2 (10022) -2%, 2000^2 (15648) 1.78 -> 1.76
@@ -300,7 +301,7 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
 inline bool merge_blocks(bool fp32, bool charac, Recon rc, bool d3, long long blocks) {
   const bool weno = rc == Recon::wenoz;
   if (fp32) return weno ? (d3 || blocks <= 16000) : blocks <= (d3 ? 40000 : 8000);
-  if (charac) return d3 && blocks <= 4500;
+  if (charac) return true;
   return blocks <= (d3 ? (weno ? 65000 : 75000) : 4500);
 }
 template <class T>
