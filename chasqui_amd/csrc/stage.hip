@@ -857,9 +857,9 @@ __global__ void __launch_bounds__(256) k_c2p(const C2pArgsT<T> a, const VB v) {
 // TURN: the fofc-branch re-run (gate 1), which ends the stage with the control turn `t`. With the
 // gate closed (nothing flagged, or the run has ended) the first block does it at once: no block
 // has work, and the turn leaves the gate closed for the others (nbad 0, `active` never set
-// again). With the gate open the last block to finish does it, counted in Ctrl::done after the
-// block's own CFL minimum has arrived (the wait); one counter limits that to FILL_TURN_TILES
-// tiles. With one turn in place of two to four control launches, ms per pass: 100 steps of a 1D
+// again). With the gate open the last block to finish does it, counted in Ctrl::done after all
+// waves of the block have read the gate, which the turn closes (the barrier), and its own CFL
+// minimum has arrived (the wait); one counter limits that to FILL_TURN_TILES tiles. With one turn in place of two to four control launches, ms per pass: 100 steps of a 1D
 // run of 128 cells 13.2 -> 11.3, 50 of 150x129 8.23 -> 7.79, 40 of 64x56x45 14.7 -> 14.4.
 template <class T, bool DT, bool TURN>
 __global__ void __launch_bounds__(256) k_fill_c2p(const C2pArgsT<T> a, const VB v, const int ngt, const CtrlTurn t) {
@@ -876,6 +876,7 @@ __global__ void __launch_bounds__(256) k_fill_c2p(const C2pArgsT<T> a, const VB 
     c2p_block_merge<DT>(a, mdt, 0, smin, ssum);
   }
   if constexpr (TURN) {
+    __syncthreads();
     if (threadIdx.x == 0) {
       __builtin_amdgcn_s_waitcnt(0);   // this thread's atomicMin is done
       if (__hip_atomic_fetch_add(&a.ctrl->done, 1, __ATOMIC_RELAXED, __HIP_MEMORY_SCOPE_AGENT) == int(gridDim.x) - 1) {
