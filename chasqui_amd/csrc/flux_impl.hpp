@@ -266,23 +266,48 @@ __global__ void __launch_bounds__(256) k_flux_x(const FluxArgsT<T> a, const int 
 }
 
 // ---------------------------------------------------------------- y/z faces: register march
-// PARK (FP32, wide stencils): what the next cell needs besides its cells' values waits in LDS while
-// the face is solved, NPARK arrays of a thread's own entries, 28 KB a block at most. The solver is
-// where the registers peak (136 to 141, three waves per SIMD); so they fit 128, four waves. ms per
-// pass: 30 steps of 192^3 PPM 144.7 -> 142.1, 20 of 128^3 WENO-Z 34.0 -> 33.6; 2D PPMX the same. In FP64
-// the same park leaves PPM and PPMX 12 to 100 bytes over three waves' 168 registers, and the spills
-// cost more than the third wave gives (256^3: 333 -> 343 ms); at two waves it only adds LDS traffic
-// (333 -> 336).
-template <class T, Recon RC> constexpr bool park_v = sizeof(T) == 4 && wide_v<RC>;
-template <Recon RC> constexpr int npark_v = RC == Recon::ppmx ? 4 : 3;
-template <class T, Recon RC, bool ENT>
-constexpr int park_n = park_v<T, RC> ? npark_v<RC> * (ENT ? 8 : 7) * BX * BY : 1;
-template <class T, Recon RC> constexpr int march_waves_v = park_v<T, RC> ? 4 : 1;
+// What a march holds besides its registers. The solver is where these peak (FP32 133 to 163, FP64 up to
+// 284 with the accumulation registers that halve the waves), so `park` of the values that only the next
+// cell needs wait in LDS while the face is solved (in this order: its left state, x1, x2, PPMX's edge;
+// a thread's own entries, 7 to 14 KB a block each), and `waves` per SIMD are asked for. ms per RK3 step:
+//   FP32, wide stencils: all parked, four waves instead of three: 192^3 PPM 4.82 -> 4.74, 128^3 WENO-Z
+//     1.70 -> 1.68; 2D PPMX the same. WENO-Z then spills 12 to 20 bytes a lane, 56 in the batched joint
+//     launch (16 runs of 128^2: 0.207, 0.304 without all of this).
+//   FP32 LHLLD holds 15 to 20 registers more. At four waves WENO-Z spills 80 to 128 bytes: three waves, two
+//     parked 64^3 0.304 -> 0.247, 128^3 1.53 -> 1.34, 224^3 7.65 -> 6.71 (6.93 before anything was parked), 1400^2
+//     0.894 -> 0.878. PPM and PPMX spill 24 to 64 and stay at four: three waves are better on small meshes and
+//     slower on others (PPM, none parked: 64^3 0.251 -> 0.232, 128^3 1.292 -> 1.298, 224^3 6.39 -> 6.22, 1400^2
+//     0.818 -> 0.838; PPMX 0.275 -> 0.263, 1.366 -> 1.419, 6.61 -> 6.62, 0.864 -> 0.883).
+//   FP64 PPM and PPMX HLLD fit two waves as they are: three leave 12 to 100 bytes over 168 registers and are
+//     slower (256^3 333 -> 343 ms per 20 steps), parking at two only adds LDS traffic (333 -> 336).
+//   FP64 PPM and PPMX with LHLLD need 4 to 10 accumulation registers, one wave: left state parked, two
+//     waves 128^3 2.63 -> 2.16 and 3.22 -> 2.45, 224^3 11.7 -> 10.3 and 14.0 -> 11.8, 512^2 0.268 -> 0.228 and
+//     0.317 -> 0.253; spilled instead 2.24 and 2.50 at 128^3. So does the batched joint PPMX launch with HLLD
+//     (16 runs of 128^2 0.356 -> 0.287).
+//   FP64 with entropy: 128^3 PPMX HLLD 3.01 -> 2.69 (left state), LHLLD 3.25 -> 2.86 (x1 too; left state alone
+//     3.04), WENO-Z LHLLD 3.40 -> 3.02 (left state). PPM peaks in the reconstruction: its fallback goes by variable
+//     (below), HLLE 2.32 -> 2.19, HLLD 2.49 -> 2.32, LHLLD 2.71 -> 2.51 with left state and x1 (one: 2.54).
+//   FP64 donor cell with LHLLD: 170 registers held to 168, three waves: 128^3 1.97 -> 1.87, 224^3 9.18 -> 8.98 (not
+//     with entropy or batched, where that spills 28 to 40 bytes).
+template <class T, Recon RC, RSolver RS, bool ENT, bool BATCH>
+struct March {
+  static constexpr bool f32 = sizeof(T) == 4, lh = RS == RSolver::lhlld, hlld = RS == RSolver::hlld;
+  static constexpr bool f32_three = lh && RC == Recon::wenoz;
+  static constexpr int fit32() { return RC == Recon::ppmx ? 4 : f32_three ? 2 : 3; }
+  static constexpr int fit64() {
+    if (RC == Recon::ppm) return lh ? (ENT ? 2 : 1) : 0;
+    if (RC == Recon::ppmx) return lh ? (ENT ? 2 : 1) : hlld && (ENT || BATCH) ? 1 : 0;
+    return lh && ENT ? 1 : 0;
+  }
+  static constexpr int park = !wide_v<RC> ? 0 : f32 ? fit32() : fit64();
+  static constexpr int waves = wide_v<RC> ? (!f32 ? 2 : f32_three ? 3 : 4)
+                                          : !f32 && RC == Recon::dc && lh && !ENT && !BATCH ? 3 : 1;
+  static constexpr int entries = park ? park * (ENT ? 8 : 7) * BX * BY : 1;
+};
 
-template <class T, int DIR, Recon RC, RSolver RS, bool ENT>
+template <class T, int DIR, Recon RC, RSolver RS, bool ENT, int PARK>
 __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx, T *park) {
   constexpr int NV = ENT ? 8 : 7, SP = BX * BY;   // SP: distance of a thread's parked entries
-  constexpr bool PARK = park_v<T, RC>;
   constexpr bool W = wide_v<RC>;
   const Geom &g = a.g;
   // i, transverse index t (k for DIR 1, j for DIR 2) and segment along DIR
@@ -371,10 +396,19 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx,
         en[n] = R::edge(w0[n], wp1[n], x1[n], dn[n], ok);    // e_{c+1/2}
         T lo = x2[n], hi = en[n];
         R::mono(w0[n], lo, hi, ok);
+        if constexpr (ENT) {   // by variable: the joint fallback takes 13 registers more (see March)
+          if (!ok) {
+            en[n] = R::template edge<true>(w0[n], wp1[n], x1[n], dn[n], ok);
+            lo = x2[n];
+            hi = en[n];
+            R::template mono<true>(w0[n], lo, hi, ok);
+            ok = true;
+          }
+        }
         Rf[n] = lo;
         Lf[n] = hi;
       }
-      if (!ok) {
+      if (!ENT && !ok) {
 #pragma unroll
         for (int n = 0; n < NV; ++n) {
           en[n] = R::template edge<true>(w0[n], wp1[n], x1[n], dn[n], ok);
@@ -412,25 +446,25 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx,
     for (int n = 0; n < NV; ++n) qc[n] = w0[n];
     finish_cell<T, NV>(Lf, Rf, qc, fco, flat, dfl, pfl);
     T *const pk = park + int(threadIdx.y) * BX + int(threadIdx.x);
-    if constexpr (PARK) {
+    if constexpr (PARK > 0) {
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         pk[n * SP] = Lf[n];
-        pk[(NV + n) * SP] = x1[n];
-        pk[(2 * NV + n) * SP] = x2[n];
-        if constexpr (RC == Recon::ppmx) pk[(3 * NV + n) * SP] = ep[n];
+        if constexpr (PARK > 1) pk[(NV + n) * SP] = x1[n];
+        if constexpr (PARK > 2) pk[(2 * NV + n) * SP] = x2[n];
+        if constexpr (PARK > 3) pk[(3 * NV + n) * SP] = ep[n];
       }
       asm volatile("" ::: "memory");   // (nothing is forwarded past the solver in registers)
     }
     if (c >= F0) solve_store<T, DIR, RS, ENT, NV>(a, cc, sd, Lprev, Rf);   // face c (between c-1 and c)
-    if constexpr (PARK) {
+    if constexpr (PARK > 0) {
       asm volatile("" ::: "memory");
 #pragma unroll
       for (int n = 0; n < NV; ++n) {
         Lf[n] = pk[n * SP];
-        x1[n] = pk[(NV + n) * SP];
-        x2[n] = pk[(2 * NV + n) * SP];
-        if constexpr (RC == Recon::ppmx) ep[n] = pk[(3 * NV + n) * SP];
+        if constexpr (PARK > 1) x1[n] = pk[(NV + n) * SP];
+        if constexpr (PARK > 2) x2[n] = pk[(2 * NV + n) * SP];
+        if constexpr (PARK > 3) ep[n] = pk[(3 * NV + n) * SP];
       }
     }
     // advance the window
@@ -447,22 +481,22 @@ __device__ __forceinline__ void flux_m_tile(const FluxArgsT<T> &a, const int bx,
 }
 
 template <class T, int DIR, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(BX * BY, (march_waves_v<T, RC>)) k_flux_m(const FluxArgsT<T> a) {
-  __shared__ T park[park_n<T, RC, ENT>];
+__global__ void __launch_bounds__(BX * BY, (March<T, RC, RS, ENT, false>::waves)) k_flux_m(const FluxArgsT<T> a) {
+  __shared__ T park[March<T, RC, RS, ENT, false>::entries];
   if (!a.ctrl->active) return;
-  flux_m_tile<T, DIR, RC, RS, ENT>(a, int(blockIdx.x), park);
+  flux_m_tile<T, DIR, RC, RS, ENT, March<T, RC, RS, ENT, false>::park>(a, int(blockIdx.x), park);
 }
 
 // All directions of a small mesh in one launch: the y and z march blocks first (the longer ones),
 // then the x blocks (flux_merge in kernels.hpp has the rule and the figures).
 template <class T, Recon RC, RSolver RS, bool ENT>
-__global__ void __launch_bounds__(256, (march_waves_v<T, RC>)) k_flux_all(const FluxArgsT<T> a0, const FluxArgsT<T> a1, const FluxArgsT<T> a2,
+__global__ void __launch_bounds__(256, (March<T, RC, RS, ENT, false>::waves)) k_flux_all(const FluxArgsT<T> a0, const FluxArgsT<T> a1, const FluxArgsT<T> a2,
                                                   const int nseg, const int nwaves, const int nby, const int nbz) {
-  __shared__ T park[park_n<T, RC, ENT>];
+  __shared__ T park[March<T, RC, RS, ENT, false>::entries];
   if (!a0.ctrl->active) return;
   const int b = int(blockIdx.x);
-  if (b < nby) flux_m_tile<T, 1, RC, RS, ENT>(a1, b, park);
-  else if (b < nby + nbz) flux_m_tile<T, 2, RC, RS, ENT>(a2, b - nby, park);
+  if (b < nby) flux_m_tile<T, 1, RC, RS, ENT, March<T, RC, RS, ENT, false>::park>(a1, b, park);
+  else if (b < nby + nbz) flux_m_tile<T, 2, RC, RS, ENT, March<T, RC, RS, ENT, false>::park>(a2, b - nby, park);
   else {
     const int wave = (b - nby - nbz) * 4 + int(threadIdx.x >> 6);
     if (wave < nwaves) flux_x_wave<T, RC, RS, ENT>(a0, nseg, wave);
@@ -634,26 +668,26 @@ __global__ void __launch_bounds__(256) kb_flux_x(const RunArgs<T> *__restrict__ 
 }
 
 template <class T, int DIR, Recon RC, RSolver RS>
-__global__ void __launch_bounds__(BX * BY, (march_waves_v<T, RC>)) kb_flux_m(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
+__global__ void __launch_bounds__(BX * BY, (March<T, RC, RS, false, true>::waves)) kb_flux_m(const RunArgs<T> *__restrict__ R, const Item *__restrict__ item,
                                                  const int *__restrict__ nitem, const int cur) {
-  __shared__ T park[park_n<T, RC, false>];
+  __shared__ T park[March<T, RC, RS, false, true>::entries];
   const int n = *nitem;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
     const Item m = uniform_item(item, it);
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][DIR];
-    flux_m_tile<T, DIR, RC, RS, false>(a, m.tile, park);
+    flux_m_tile<T, DIR, RC, RS, false, March<T, RC, RS, false, true>::park>(a, m.tile, park);
   }
 }
 
 // All directions of a batch with little work in one launch, in the order of k_flux_all.
 template <class T, Recon RC, RSolver RS>
-__global__ void __launch_bounds__(256, (march_waves_v<T, RC>)) kb_flux_all(
+__global__ void __launch_bounds__(256, (March<T, RC, RS, false, true>::waves)) kb_flux_all(
     const RunArgs<T> *__restrict__ R, const Item *__restrict__ item0, const Item *__restrict__ item1,
     const Item *__restrict__ item2, const int *__restrict__ n0, const int *__restrict__ n1, const int *__restrict__ n2,
     const int cur) {
-  __shared__ T park[park_n<T, RC, false>];
+  __shared__ T park[March<T, RC, RS, false, true>::entries];
   const int ny = *n1, nz = *n2, n = ny + nz + *n0;
   for (int it = int(blockIdx.x); it < n; it += int(gridDim.x)) {
     const int dir = it < ny ? 1 : it < ny + nz ? 2 : 0;
@@ -662,8 +696,8 @@ __global__ void __launch_bounds__(256, (march_waves_v<T, RC>)) kb_flux_all(
     const Ctrl *ctl = R[m.run].ctrl;
     if (!ctl->active) continue;
     const FluxArgsT<T> a = R[m.run].flux[cur][uniform(ctl->wcur)][dir];
-    if (dir == 1) flux_m_tile<T, 1, RC, RS, false>(a, m.tile, park);
-    else if (dir == 2) flux_m_tile<T, 2, RC, RS, false>(a, m.tile, park);
+    if (dir == 1) flux_m_tile<T, 1, RC, RS, false, March<T, RC, RS, false, true>::park>(a, m.tile, park);
+    else if (dir == 2) flux_m_tile<T, 2, RC, RS, false, March<T, RC, RS, false, true>::park>(a, m.tile, park);
     else {
       int nseg, nwaves;
       x_shape(a, fpw_v<RC>, nseg, nwaves);
