@@ -377,9 +377,11 @@ __device__ __forceinline__ void update_at_loop(const UpdateArgsT<T> &a, const do
 // Stamps of earlier stages hold smaller epochs and are ignored. With the stamps in the repair's
 // launch and both re-updates in one, a stage of this kind has two launches fewer (about 4 us each
 // on the device even when nothing was flagged).
-template <class T>
-__global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, const CornerArgsT<T> ca, const int corn,
-                                                     const VB v, const int *marks) {
+// Most points only read their mark, so the launch lives on the waves in flight: the form without the
+// edge EMFs is a kernel of its own (25 VGPRs in FP64, 19 in FP32, seven waves per SIMD; with the 1D and 2D
+// form beside it 128 and 109, four waves: the firing launch at 256^3 77 us in place of 54 and 75 in place of 53).
+template <class T, class F>
+__device__ __forceinline__ void near_walk(const UpdateArgsT<T> &a, const VB &v, const int *marks, F update) {
   if (!gate(a.ctrl, 1)) return;
   const Geom &g = a.g;
   const double bdt = a.use_ctrl_dt ? a.beta * a.ctrl->dt : a.beta_dt;
@@ -389,10 +391,18 @@ __global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, con
     int k, j, i;
     if (!v.at(vb, k, j, i)) continue;
     k += g.ks; j += g.js; i += g.is;
-    if (!whole && marks[g.at(k, j, i)] != epoch) continue;
-    if (corn) update_at12<T, true>(a, ca, bdt, k, j, i);
-    else update_at_loop(a, bdt, k, j, i);
+    if (whole || marks[g.at(k, j, i)] == epoch) update(bdt, k, j, i);
   }
+}
+template <class T>
+__global__ void __launch_bounds__(256) k_update_near(const UpdateArgsT<T> a, const VB v, const int *marks) {
+  near_walk(a, v, marks, [&](double bdt, int k, int j, int i) { update_at_loop(a, bdt, k, j, i); });
+}
+// with the edge EMFs in the same thread (update_has_corner)
+template <class T>
+__global__ void __launch_bounds__(256) k_update_near12(const UpdateArgsT<T> a, const CornerArgsT<T> ca, const VB v,
+                                                       const int *marks) {
+  near_walk(a, v, marks, [&](double bdt, int k, int j, int i) { update_at12<T, true>(a, ca, bdt, k, j, i); });
 }
 
 template <class T>
@@ -1245,8 +1255,9 @@ template hipError_t launch_update<float>(const UpdateArgsT<float> &, hipStream_t
 template <class T>
 hipError_t launch_update_near(const UpdateArgsT<T> &a, const CornerArgsT<T> *ca, const int *marks, hipStream_t s) {
   const VB v = update_vb(a.g);   // a capped grid-stride grid: most points only read their mark
-  hipLaunchKernelGGL(k_update_near<T>, dim3(grid_of(v, true)), dim3(256), 0, s, a, ca ? *ca : CornerArgsT<T>{},
-                     ca ? 1 : 0, v, marks);
+  const dim3 grid(grid_of(v, true)), block(256);
+  if (ca) hipLaunchKernelGGL(k_update_near12<T>, grid, block, 0, s, a, *ca, v, marks);
+  else hipLaunchKernelGGL(k_update_near<T>, grid, block, 0, s, a, v, marks);
   return hipGetLastError();
 }
 template hipError_t launch_update_near<double>(const UpdateArgsT<double> &, const CornerArgsT<double> *, const int *, hipStream_t);

@@ -1,7 +1,12 @@
-"""The con2prim launch that ends a stage with its control turn: the last block to count itself done
+"""What the device listing of the stage kernels' source has to show.
+
+The con2prim launch that ends a stage with its control turn: the last block to count itself done
 closes the gate that every wave of the launch reads first, so a block may count itself only when
-all its waves have read it. Checked on the device listing of the source: in every such kernel no
-path from the entry reaches the count without a block barrier."""
+all its waves have read it. In every such kernel no path from the entry reaches the count without
+a block barrier.
+
+The local fofc re-update of a 3D mesh only reads a mark at most points, so it needs the waves in
+flight that a small register count gives it."""
 import os
 import re
 import shutil
@@ -44,30 +49,47 @@ def test_walk_finds_the_path_around_a_barrier():
     assert _reaches(around, lambda s: "atomic" in s) and not _reaches(through, lambda s: "atomic" in s)
 
 
-def test_no_block_counts_itself_before_all_its_waves_read_the_gate(tmp_path):
+@pytest.fixture(scope="module")
+def kernels(tmp_path_factory):
+    """Kernel name -> lines of its listing, the figures after its end included."""
     if not os.path.exists(HIPCC) and not shutil.which("hipcc"):
         pytest.skip("hipcc not available")
-    src = tmp_path / "off.cpp"
-    src.write_text('#include <cstddef>\n#include <cstdio>\n#include <hip/hip_runtime.h>\n#include "common.hpp"\n'
-                   'int main() { std::printf("%zu", offsetof(chq::Ctrl, done)); }\n')
-    exe, lst = tmp_path / "off", tmp_path / "stage.s"
-    subprocess.run([HIPCC, "--offload-host-only", *INC, str(src), "-o", str(exe)], check=True, capture_output=True)
-    off = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+    lst = tmp_path_factory.mktemp("stage") / "stage.s"
     subprocess.run([HIPCC, "--offload-arch=gfx950", "--offload-device-only", "-S", "-O3", "-ffp-contract=off", "-Xclang",
                     "-target-feature", "-Xclang", "-packed-fp32-ops", *INC,
                     os.path.join(ROOT, "chasqui_amd", "csrc", "stage.hip"), "-o", str(lst)], check=True, capture_output=True)
-    kernels, name = {}, None
+    out, name = {}, None
     for s in lst.read_text().splitlines():
-        m = re.match(r"(_Z\S*k_fill_c2pI[df]Lb[01]ELb1EE\S*):", s)   # <T, DT, TURN = true>
+        m = re.match(r"(_Z\w+):", s)
         if m:
             name = m.group(1)
-        elif s.startswith(".Lfunc_end"):
-            name = None
         if name:
-            kernels.setdefault(name, []).append(s)
-    assert len(kernels) == 4, sorted(kernels)
-    for name, lines in kernels.items():
-        def count(s):
-            return s.startswith("global_atomic_add ") and s.endswith("offset:" + off + " sc0")
+            out.setdefault(name, []).append(s)
+    return out
+
+
+def test_no_block_counts_itself_before_all_its_waves_read_the_gate(tmp_path, kernels):
+    src, exe = tmp_path / "off.cpp", tmp_path / "off"
+    src.write_text('#include <cstddef>\n#include <cstdio>\n#include <hip/hip_runtime.h>\n#include "common.hpp"\n'
+                   'int main() { std::printf("%zu", offsetof(chq::Ctrl, done)); }\n')
+    subprocess.run([HIPCC, "--offload-host-only", *INC, str(src), "-o", str(exe)], check=True, capture_output=True)
+    off = subprocess.run([str(exe)], capture_output=True, text=True, check=True).stdout
+
+    def count(s):
+        return s.startswith("global_atomic_add ") and s.endswith("offset:" + off + " sc0")
+
+    turn = [k for k in kernels if re.search(r"k_fill_c2pI[df]Lb[01]ELb1EE", k)]   # <T, DT, TURN = true>
+    assert len(turn) == 4, turn
+    for name in turn:
+        lines = [s for s in kernels[name]]
+        lines = lines[:next(n for n, s in enumerate(lines) if s.startswith(".Lfunc_end"))]
         assert sum(count(s.split(";")[0].strip()) for s in lines) == 1, name
         assert not _reaches(lines, count), name
+
+
+def test_local_reupdate_of_3d_meshes_keeps_its_waves(kernels):
+    near = [k for k in kernels if re.search(r"k_update_nearI[df]E", k)]
+    assert len(near) == 2, near
+    for name in near:
+        occ = [int(m.group(1)) for s in kernels[name] if (m := re.match(r"; Occupancy: (\d+)", s))]
+        assert occ and occ[0] >= 7, (name, occ)
