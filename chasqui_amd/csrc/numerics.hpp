@@ -122,10 +122,13 @@ template <class T> struct Rec {
       const T cap = T(2) * vmin(vabs(l), vabs(r));
       return sgn(m) * vmin(vabs(m), cap);
     }
-    // where the product is positive m is not zero, so copysign is the reference's sgn(m) * (...)
-    const T m = T(0.5) * (c - a);
+    // Without the branch. Where the product is not <= 0, m is zero only as an exact +0, with a zero to
+    // scale, so a sign bit is the reference's sgn(m); a NaN m (its sgn is 0) and a NaN product (infinite
+    // neighbours) give what the reference gives. The branch instead: 64x56x45 0.251 -> 0.255 ms per
+    // step, 128^3 2.00 -> 2.01; a plain copysign, wrong beside two infinite values: 0.250 and 1.99.
+    const T m = T(0.5) * (c - a), s = m == m ? vcopysign(T(1), m) : T(0);
     const T cap = T(2) * vmin(vabs(l), vabs(r));
-    return l * r > T(0) ? vcopysign(vmin(vabs(m), cap), m) : T(0);
+    return l * r <= T(0) ? T(0) : s * vmin(vabs(m), cap);
   }
   // The FP64 CW84 steps hold one branch per cell and variable (the extremum test, which lets the
   // waves of a uniform region leave early) instead of six: a divergent branch costs the wave its
