@@ -260,7 +260,7 @@ struct Batch final : BatchBase {
     const int *g = b->grid;
     if (merge) {
       const ItemList fl[3] = {list(K_FLUX1), list(K_FLUX2), list(K_FLUX3)};
-      HIPCHK(launchb_flux_all(d_runs, fl, cf.cur, rc, rs, std::max({g[K_FLUX1], g[K_FLUX2], g[K_FLUX3]}), st));
+      HIPCHK(launchb_flux_all(d_runs, fl, cf.cur, rc, rs, g[K_FLUX1], st));
     }
     for (int d = 0; d < 3; ++d)
       if (present[K_FLUX1 + d] && !merge) HIPCHK(launchb_flux(d_runs, list(K_FLUX1 + d), d, cf.cur, rc, rs, g[K_FLUX1 + d], st));
@@ -326,7 +326,12 @@ struct Batch final : BatchBase {
     hipStream_t st = b->stream;
     switch (q) {
       case K_FLUX1: case K_FLUX2: case K_FLUX3:
-        HIPCHK(launchb_flux(d_runs, list(q), q - K_FLUX1, 0, rc, rs, gsz, st));
+        if (merge) {
+          const ItemList fl[3] = {list(K_FLUX1), list(K_FLUX2), list(K_FLUX3)};
+          HIPCHK(launchb_flux_all(d_runs, fl, 0, rc, rs, gsz, st));
+        } else {
+          HIPCHK(launchb_flux(d_runs, list(q), q - K_FLUX1, 0, rc, rs, gsz, st));
+        }
         break;
       case K_CORNER: HIPCHK(launchb_corner<T>(d_runs, list(q), gsz, st)); break;
       case K_UPDATE: HIPCHK(launchb_update<T>(d_runs, list(q), 1, 1.0, 0.0, 1.0, gsz, st)); break;
@@ -352,11 +357,14 @@ struct Batch final : BatchBase {
       HIPCHK(hipMemcpyAsync(d_runs, h_runs.data(), sizeof(RunArgs<T>) * h_runs.size(), hipMemcpyHostToDevice, b->stream));
     double total = 0.0;
     for (int q = 0; q < K_NLIST; ++q) {
-      if (h_count[1 + q] == 0) continue;
+      int items = h_count[1 + q];
+      if (merge && q <= K_FLUX3)   // one launch for the lists of all directions, with flux_x1's grid
+        items = q == K_FLUX1 ? h_count[1 + K_FLUX1] + h_count[1 + K_FLUX2] + h_count[1 + K_FLUX3] : 0;
+      if (items == 0) continue;
       double best = 1e30;
       int best_g = b->grid[q];
       for (int gsz : cand) {
-        if (gsz > 4 * h_count[1 + q] && gsz > 256) break;
+        if (gsz > 4 * items && gsz > 256) break;
         if (int e = launch_class(q, gsz)) return e;   // warm
         std::vector<float> t;
         for (int rep = 0; rep < reps; ++rep) {

@@ -264,7 +264,9 @@ int chq_batch_use_graph(chq_batch *batch, int on);     /* default on */
  * configuration; touches only arrays a step rewrites) and keeps the fastest; best_ms = sum of
  * the best per-class launch times. Call between steps. */
 int chq_batch_tune(chq_batch *batch, int reps, double *best_ms);
-/* grid size (blocks) of kernel class `cls` (0..10) and its name */
+/* grid size (blocks) of kernel class `cls` (0..10) and its name. Batches whose face fluxes go in
+ * one launch for all directions use flux_x1's for it; bc_x1..bc_x3 have no launch (the ghost fill
+ * is part of c2p's). */
 int chq_batch_grid(chq_batch *batch, int cls, int *grid, const char **name);
 int chq_batch_set_grid(chq_batch *batch, int cls, int grid);
 
