@@ -200,17 +200,18 @@ constexpr int BX = 64, BY = 4;
 // Faces per thread in the y/z march. A thread of a segment of s faces reconstructs s + 1 cells and
 // solves s faces one after the other: long segments save the extra reconstruction, short ones
 // give a small launch more waves and a shorter serial chain. march_seg picks the candidate of
-// least cost (s + 0.7) (0.1 + 0.9 m), where m is the launch's 256-thread blocks per CU (a block
+// least cost (s + 0.9) (0.15 + 0.85 m), where m is the launch's 256-thread blocks per CU (a block
 // puts one wave on each SIMD of its CU, and the waves of a SIMD share its issue slots, so the
-// second block of a CU adds nine tenths of the first one's time); a partial last block per CU
-// counts three quarters of a whole one. The three constants are fitted to sweeps of the RK step
-// over segments of 1 to 32 on 64^2 .. 1024^2 and 32^3 .. 192^3, PLM, PPM, PPMX, WENO-Z and
-// characteristic PPMX, both precisions: the choice is within 0.5% of the best candidate on
-// average (5% at worst). Before (24 faces where the march threads fill the device, 8 below, 4
-// below a sixteenth of it), ms per RK3 step: 150x129 PPMX FP64 0.233 (now 0.187), 64x56x45 PPM
-// FP64 0.495 (0.396), 512^2 PPMX mixed 0.298 (0.258), 80x72x64 characteristic 1.089 (the same segment),
-// 128^3 PPM FP64 2.301 (2.249). The choice moves work between threads only: every face is
-// computed by the same expressions either way.
+// second block of a CU adds 0.85 of the first one's time); a partial last block per CU counts
+// half as such and half as a whole one. The three constants are fitted to sweeps over segments of
+// 1 to 24 of the meshes whose directions have a launch each (dual energy, explicit diffusion, the
+// sizes beyond flux_merge's limits): 64^3 .. 240^3 and 200^2 .. 2200^2, PLM, PPM, PPMX, WENO-Z,
+// both precisions: the choice is within 0.5% of the best candidate on average (4.3% at worst, 600^2
+// of PPMX LHLLD; else 2.5%). (s + 0.7) (0.1 + 0.9 m) with three quarters of a whole block for the
+// partial one gave 0.8% and 6.6%: 144^3 took 3 faces (now 8; ms per step of dual energy PPMX 3.78 ->
+// 3.61, WENO-Z 4.02 -> 3.86, PPM with explicit diffusion 4.65 -> 4.54; 4.62 with the 24 faces it had
+// before any model). The choice moves work between threads only: every face is computed by the same
+// expressions either way.
 struct MarchShape {
   long long rows;   // threads per segment layer: the face range across the march direction
   int nd;           // faces along it
@@ -233,8 +234,8 @@ inline int march_seg(const MarchShape *sh, int n) {
       len = len > sh[q].nd ? len : sh[q].nd;
     }
     const double per = double(blocks) / 256.0;   // 256 CUs
-    const double m = 0.75 * double((blocks + 255) / 256) + 0.25 * per;
-    const double cost = ((s < len ? s : len) + 0.7) * (0.1 + 0.9 * (m > 1.0 ? m : 1.0));
+    const double m = 0.5 * double((blocks + 255) / 256) + 0.5 * per;
+    const double cost = ((s < len ? s : len) + 0.9) * (0.15 + 0.85 * (m > 1.0 ? m : 1.0));
     if (cost < least) { least = cost; best = s; }
   }
   return best;
