@@ -97,7 +97,6 @@ __device__ __forceinline__ void eigen_of(double d, double p, double by, double b
   E.l6[1] = ncff; E.l6[2] = -nqs * bety; E.l6[3] = -nqs * betz; E.l6[4] = norm * alf / d; E.l6[5] = nas * bety; E.l6[6] = nas * betz;
 }
 
-// characteristic variable KK of one stencil point: sum_n L[KK][n] q[n], ascending n, from +0
 // The 7 or 8 variables of one window cell in LDS, a thread's entries SP apart.
 struct Parked {
   static constexpr int SP = BX * BY;
@@ -106,6 +105,7 @@ struct Parked {
   __device__ __forceinline__ void set(int n, double v) const { p[n * SP] = v; }
 };
 
+// characteristic variable KK of one stencil point: sum_n L[KK][n] q[n], ascending n, from +0
 template <int KK, class Q>
 __device__ __forceinline__ double project(const Eig &E, const Q &q) {
   double acc = 0.0;

@@ -296,7 +296,8 @@ __host__ __device__ inline bool m_item(const FluxArgsT<T> &a, long long lin, int
 //          characteristic PPMX (x kernel and march both at two waves): 80x72x64 (3083) 1.087 -> 1.009, 96^3 (7278)
 //                 -8%, 112^3 -4%, 144^3 (24145) -7%; 200^2 -16%, 500^2 -11%: always
 //   FP32   PPM    144^3 (24145) -3.5%, 192^3 (56748) -2.2% for a wave but 30 steps of a blast +0.6%, 240^3 -0.2%, PPMX
-//                 there +1.3%; 1300^2 (6616) -1.9%, 1600^2 +0.6%; PLM 192^3 +0.3%
+//                 there +1.3%; 1300^2 (6616) -1.9%, 1600^2 +0.6%; PLM 192^3 +0.3%. The 3D limit is what the
+//                 blast allows: a wave alone would take one launch at 192^3 too.
 //          WENO-Z 192^3 -2.1%, 256^3 (133648) 9.62 -> 9.41; 1600^2 (10022) -2%, 2000^2 (15648) 1.78 -> 1.76
 // A batch counts the march blocks of all its runs (64 small mixed runs 28.4 -> 26.6 ms per 100 steps).
 inline bool merge_blocks(bool fp32, bool charac, Recon rc, bool d3, long long blocks) {

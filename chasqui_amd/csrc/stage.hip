@@ -847,10 +847,12 @@ __device__ __forceinline__ void ctrl_turn(Ctrl *c, const CtrlTurn &t) {
 // k_c2p: u[IENT] is transported or stored, ghosts filled by a launch before (k_fill).
 // k_fill_c2p: the fast path, with the ghost fill in the same launch. A dependent launch costs about
 // 4.5 us on the device even when it does nothing, and the x1 fill alone touches two lines per row
-// and array for three values (23 us at 192^3); behind the active tiles both are hidden. Against a
-// launch per direction and then con2prim over all cells, ms per pass: 50 steps of 150x129 9.76 ->
-// 8.23, 50 of 512^2 mixed 14.3 -> 12.6, 40 of 64x56x45 16.8 -> 14.7, 20 of 256^3 338 -> 332, 100 of
-// 64 small mixed runs 33.5 -> 30.0. Active rows are also whole lines, which rows with ghosts are not.
+// and array for three values (23 us at 192^3). In FP64 both are hidden behind the active tiles (256^3:
+// 654 us, con2prim alone 654 and the three fills 89 before); a large mixed mesh only saves the
+// launches (552 us, before 464 and 89). Against a launch per direction and then con2prim over all
+// cells, ms per pass: 50 steps of 150x129 9.76 -> 8.23, 50 of 512^2 mixed 14.3 -> 12.6, 40 of 64x56x45
+// 16.8 -> 14.7, 20 of 256^3 338 -> 332, 100 of 64 small mixed runs 33.5 -> 30.0. FP64 active rows are
+// also whole lines, which rows with ghosts are not.
 template <class T, bool DT, bool DE>
 __global__ void __launch_bounds__(256) k_c2p(const C2pArgsT<T> a, const VB v) {
   if (!gate(a.ctrl, a.only_if_bad)) return;
